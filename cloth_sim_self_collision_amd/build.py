@@ -21,9 +21,11 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libclothsim.so")
 BUILD_DIR = os.path.join(HERE, "_build")
 
-SOURCES = ["cs_setup.cpp", "cs_setup_cache.cpp", "cs_api.cpp", "cs_solve.hip", "cs_contact.hip",
+SOURCES = ["cs_setup.cpp", "cs_setup_cache.cpp", "cs_strips.cpp", "cs_api.cpp", "cs_solve.hip",
+           "cs_strips.hip", "cs_contact.hip",
            "cs_elements.hip", "cs_noalloc.hip"]
-HEADERS = ["cs_math.hpp", "cs_ordered_sum.hpp", "cs_setup.hpp", "cs_device.hpp", "cs_solve.hpp", "cs_contact.hpp"]
+HEADERS = ["cs_math.hpp", "cs_ordered_sum.hpp", "cs_setup.hpp", "cs_strips.hpp",
+           "cs_device.hpp", "cs_solve.hpp", "cs_contact.hpp"]
 
 ARCH = os.environ.get("CLOTHSIM_ARCH", "gfx950")
 FLAGS = [

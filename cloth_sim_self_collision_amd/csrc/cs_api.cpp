@@ -18,6 +18,7 @@
 #include "cs_device.hpp"
 #include "cs_setup.hpp"
 #include "cs_solve.hpp"
+#include "cs_strips.hpp"
 
 namespace cs {
 
@@ -146,6 +147,7 @@ struct Cloth {
   ContactState contact;
   bool have_x1 = false;
   int poll = 8;
+  int packed = 0;  // packed copies of the current factor (Packed)
   Prof prof;
   double time = 0.0;  // simulated time, advanced by dt per cs_step
   // kinematic sweep: vertices placed at rest + delta * clamp((t+dt)/duration, 0, 1)
@@ -312,6 +314,23 @@ int build(Cloth* c, const cs_mesh* m) {
   int *qfc, *qbc;
   A.reserve(&qfc, S.qf_comp.size());
   A.reserve(&qbc, S.qb_comp.size());
+  StripPlan T;
+  build_strips(S, T);
+  // the records are addressed with 32-bit byte offsets inside a result array
+  if (24LL * np >= (1LL << 31) || 512LL * T.bwd.nsub >= (1LL << 31)) T.ok = false;
+  int *stfp, *stbp, *stfs, *stbs, *stfr, *stbr, *stsl;
+  const size_t nsf = T.ok ? T.fwd.nsub + kStripTail : 0, nsb = T.ok ? T.bwd.nsub + kStripTail : 0;
+  A.reserve(&stfp, T.fwd.ptr.size());
+  A.reserve(&stbp, T.bwd.ptr.size());
+  A.reserve(&stfs, 64 * nsf);
+  A.reserve(&stbs, 64 * nsb);
+  A.reserve(&stfr, kStripRows * nsf);
+  A.reserve(&stbr, kStripRows * nsb);
+  A.reserve(&stsl, T.ok ? (size_t)np : 0);
+  A.reserve(&d.st_frec, strip_record_bytes(true, T.k) * nsf);
+  A.reserve(&d.st_brec, strip_record_bytes(false, T.k) * nsb);
+  A.reserve(&d.st_sb, 64 * nsb);
+  A.reserve(&d.st_ticket, 1);
   double* host_pd;
   A.reserve(&host_pd, 4 * (size_t)np);
   if (int st = A.commit(c->stream)) return st;
@@ -370,6 +389,49 @@ int build(Cloth* c, const cs_mesh* m) {
   d.ncomp = S.ncomp;
   d.qwidth = S.qwidth;
   hipStream_t s = c->stream;
+  if (T.ok) {
+    d.st_nf = (int)T.fwd.ptr.size() - 1;
+    d.st_nb = (int)T.bwd.ptr.size() - 1;
+    d.st_nsf = T.fwd.nsub;
+    d.st_nsb = T.bwd.nsub;
+    d.st_ring = T.ring;
+    d.st_fptr = stfp;
+    d.st_bptr = stbp;
+    d.st_fsrc = stfs;
+    d.st_bsrc = stbs;
+    d.st_frow = stfr;
+    d.st_brow = stbr;
+    d.st_fslot = stsl;
+    d.st_fstride = strip_record_bytes(true, T.k);
+    d.st_rhs_off = strip_rhs_offset(T.k);
+    if (int st = upload(stfp, T.fwd.ptr, s)) return st;
+    if (int st = upload(stbp, T.bwd.ptr, s)) return st;
+    if (int st = upload(stfr, T.fwd.row, s)) return st;
+    if (int st = upload(stbr, T.bwd.row, s)) return st;
+    if (int st = upload(stsl, T.fwd.slot, s)) return st;
+    // the plan's arrays only pass through (the backward slots, then each
+    // sweep's ring offsets and imports)
+    void* tmp = nullptr;
+    const size_t nslot = sizeof(int) * np;
+    const size_t ncol = sizeof(unsigned short) * std::max(T.fwd.col.size(), T.bwd.col.size());
+    const size_t col_at = (nslot + 255) / 256 * 256, imp_at = col_at + (ncol + 255) / 256 * 256;
+    if (int st = dev_alloc(&tmp, imp_at + sizeof(int) * std::max(T.fwd.import.size(),
+                                                                 T.bwd.import.size()), s))
+      return st;
+    int* bslot = (int*)tmp;
+    unsigned short* col = (unsigned short*)((char*)tmp + col_at);
+    int* import = (int*)((char*)tmp + imp_at);
+    int st = upload(bslot, T.bwd.slot, s);
+    for (int dir = 0; dir < 2 && st == kOk; dir++) {
+      const StripSweep& w = dir == 0 ? T.fwd : T.bwd;
+      st = upload(col, w.col, s);
+      if (st == kOk) st = upload(import, w.import, s);
+      if (st == kOk) st = launch_strip_meta(d, dir == 0, col, import, bslot, s);
+    }
+    dev_free(tmp, s);
+    if (st != kOk) return st;
+    if (int st = launch_strip_reset(d, s)) return st;
+  }
   CS_HIP(hipMemsetAsync(d.sum.ticket, 0, sizeof(unsigned int), s));
   CS_HIP(hipMemsetAsync(d.sum2.ticket, 0, sizeof(unsigned int), s));
   CS_HIP(hipMemcpyAsync(tri, m->tri, sizeof(int) * 3 * nt, hipMemcpyHostToDevice, s));
@@ -451,8 +513,15 @@ int sync(Cloth* c) {
   return kOk;
 }
 
-int check_tickets(const int* hflags) {
-  if (hflags[kTicketErr]) {
+// the flags of a finished solve (in c->hflags): its reductions and sweeps ended
+// as they must
+int check_solve(Cloth* c) {
+  if (c->hflags[kSweepErr]) {
+    set_error("a strip of an ILU sweep gave up waiting for the strip before it");
+    (void)launch_strip_reset(c->d, c->stream);
+    return kHipError;
+  }
+  if (c->hflags[kTicketErr]) {
     set_error("a PCG reduction ended with its ticket nonzero (inconsistent skip flag)");
     return kHipError;
   }
@@ -468,13 +537,15 @@ int internal_step(Cloth* c, double* conv, int* iters) {
   Prof* prof = c->prof.on ? &c->prof : nullptr;
   if (int st = launch_assemble(d, c->P, s, prof)) return st;
   if (int st = launch_ilu(d, s, prof)) return st;
-  if (int st = run_pcg(d, c->P.pcg_tol, c->P.pcg_maxit, c->hflags, s, c->poll, prof, &c->aux))
+  c->packed = 0;
+  if (int st = run_pcg(d, c->P.pcg_tol, c->P.pcg_maxit, c->hflags, &c->packed, s, c->poll, prof,
+                       &c->aux))
     return st;
   if (int st = launch_finish_internal(d, c->P, s)) return st;
   CS_HIP(hipMemcpyAsync(c->hflags, d.flags, sizeof(int) * kNumFlag, hipMemcpyDeviceToHost, s));
   CS_HIP(hipMemcpyAsync(c->hscal, d.scal, sizeof(double) * kNumScal, hipMemcpyDeviceToHost, s));
   CS_HIP(hipStreamSynchronize(s));
-  if (int st = check_tickets(c->hflags)) return st;
+  if (int st = check_solve(c)) return st;
   if (conv) *conv = c->hscal[kConv];
   if (iters) *iters = c->hflags[kDone] ? c->hflags[kIters] : c->P.pcg_maxit;
   if (c->hflags[kFlagNonFinite]) {
@@ -774,9 +845,8 @@ int cs_set_option(cs_cloth* p, int option, int value) {
       return kBadArg;
     }
     c->d.precision = value;
-    // the packed coefficients change format: repack the current factor
-    if (int st = launch_pack_factor(c->d, c->stream)) return st;
-    return sync(c);
+    c->packed = 0;  // the packed coefficients change format
+    return kOk;
   }
   set_error("unknown option or value");
   return kBadArg;
@@ -878,6 +948,7 @@ int cs_ilu_factor(cs_cloth* p, int* n_singular) {
   Cloth* c = H(p);
   CS_HIP(hipMemsetAsync(c->d.flags, 0, sizeof(int) * kNumFlag, c->stream));
   if (int st = launch_ilu(c->d, c->stream)) return st;
+  c->packed = 0;
   CS_HIP(hipMemcpyAsync(c->hflags, c->d.flags, sizeof(int) * kNumFlag, hipMemcpyDeviceToHost, c->stream));
   if (int st = sync(c)) return st;
   if (n_singular) *n_singular = c->hflags[kNsing];
@@ -901,7 +972,7 @@ int cs_set_factor(cs_cloth* p, const double* fdia, const double* fcrs) {
   if (fdia) CS_HIP(hipMemcpyAsync(c->d.fdia, fdia, sizeof(double) * 9 * c->S.np, hipMemcpyHostToDevice, s));
   if (fcrs && c->S.nnz)
     CS_HIP(hipMemcpyAsync(c->d.fcrs, fcrs, sizeof(double) * 9 * c->S.nnz, hipMemcpyHostToDevice, s));
-  if (int st = launch_pack_factor(c->d, s)) return st;
+  c->packed = 0;
   return sync(c);
 }
 
@@ -912,9 +983,11 @@ int cs_ilu_solve(cs_cloth* p, double* vec) {
   const size_t n = sizeof(double) * 3 * c->S.np;
   CS_HIP(hipMemsetAsync(c->d.flags, 0, sizeof(int) * kNumFlag, s));
   CS_HIP(hipMemcpyAsync(c->d.r, vec, n, hipMemcpyHostToDevice, s));
-  if (int st = launch_ilu_apply(c->d, c->d.r, c->d.z, s)) return st;
+  if (int st = launch_ilu_apply(c->d, c->d.r, c->d.z, &c->packed, s)) return st;
   CS_HIP(hipMemcpyAsync(vec, c->d.z, n, hipMemcpyDeviceToHost, s));
-  return sync(c);
+  CS_HIP(hipMemcpyAsync(c->hflags, c->d.flags, sizeof(int) * kNumFlag, hipMemcpyDeviceToHost, s));
+  if (int st = sync(c)) return st;
+  return check_solve(c);
 }
 
 int cs_matvec(cs_cloth* p, double alpha, const double* x, double beta, double* y) {
@@ -936,13 +1009,14 @@ int cs_pcg_solve(cs_cloth* p, const double* b, double tol, int maxit, double* x,
   hipStream_t s = c->stream;
   const size_t n = sizeof(double) * 3 * c->S.np;
   CS_HIP(hipMemcpyAsync(c->d.b, b, n, hipMemcpyHostToDevice, s));
-  if (int st = run_pcg(c->d, tol, maxit, c->hflags, s, c->poll, nullptr, &c->aux)) return st;
+  if (int st = run_pcg(c->d, tol, maxit, c->hflags, &c->packed, s, c->poll, nullptr, &c->aux))
+    return st;
   if (x) CS_HIP(hipMemcpyAsync(x, c->d.dx, n, hipMemcpyDeviceToHost, s));
   if (r) CS_HIP(hipMemcpyAsync(r, c->d.r, n, hipMemcpyDeviceToHost, s));
   CS_HIP(hipMemcpyAsync(c->hflags, c->d.flags, sizeof(int) * kNumFlag, hipMemcpyDeviceToHost, s));
   CS_HIP(hipMemcpyAsync(c->hscal, c->d.scal, sizeof(double) * kNumScal, hipMemcpyDeviceToHost, s));
   if (int st = sync(c)) return st;
-  if (int st = check_tickets(c->hflags)) return st;
+  if (int st = check_solve(c)) return st;
   if (conv) *conv = c->hscal[kConv];
   if (iters) *iters = c->hflags[kDone] ? c->hflags[kIters] : maxit;
   return kOk;
@@ -1193,6 +1267,9 @@ extern "C" int cs_batch_create(int n, cs_cloth* const* cloths, cs_batch** out) {
                           ? -1
                           : std::max(v.max_fu_blocks, d.fu_blocks);
     v.piped = v.piped && quad_ok(d) && (v.kpack == 0 || v.kpack == d.kpack);
+    v.max_strips = std::max(v.max_strips, std::max(d.st_nf, d.st_nb));
+    v.max_ring = std::max(v.max_ring, d.st_ring);
+    v.max_subs = std::max(v.max_subs, d.st_nsf + d.st_nsb);
     v.kpack = d.kpack;
   }
   v.wg = v.piped;
@@ -1277,6 +1354,8 @@ extern "C" int cs_batch_step(cs_batch* p, int nsteps, cs_step_stats* stats) {
   // same either way): the one-workgroup solve when every member selects it
   b->view.wg = b->view.piped;
   for (Cloth* c : b->cl) b->view.wg = b->view.wg && pcg_wg_ok(c->d) && c->d.pcg_variant == 2;
+  b->view.strips = b->view.piped;
+  for (Cloth* c : b->cl) b->view.strips = b->view.strips && strips_ok(c->d);
   // one sweep instance serves every member: their coefficient formats agree
   b->view.f32 = b->cl[0]->d.precision != 0;
   for (Cloth* c : b->cl)
@@ -1294,16 +1373,18 @@ extern "C" int cs_batch_step(cs_batch* p, int nsteps, cs_step_stats* stats) {
                                c->sweep_delta[2] * sv};
         if (int st = launch_apply_sweep(c->d, c->sweep_verts, c->n_sweep, off, s)) return st;
       }
+    for (Cloth* c : b->cl) c->packed = 0;  // the step makes new factors
     if (int st = batch_internal_step(b->view, b->tol, b->maxit, b->poll, b->dgather, b->hgather, s,
                                      b->prof.on ? &b->prof : nullptr, &b->aux))
       return st;
     for (Cloth* c : b->cl) {
+      c->packed = b->view.strips && !b->view.wg ? kPackedStrips : kPackedQuad;
       CS_HIP(hipMemcpyAsync(c->hflags, c->d.flags, sizeof(int) * kNumFlag, hipMemcpyDeviceToHost, s));
       CS_HIP(hipMemcpyAsync(c->hscal, c->d.scal, sizeof(double) * kNumScal, hipMemcpyDeviceToHost, s));
     }
     CS_HIP(hipStreamSynchronize(s));
     for (size_t i = 0; i < n; i++)
-      if (int st = check_tickets(b->cl[i]->hflags)) return st;
+      if (int st = check_solve(b->cl[i])) return st;
     // contact passes: every cloth on its own stream, from up to
     // kContactThreads host threads (each pass waits on the host for its
     // contact counts, so passes of different cloths overlap those waits)

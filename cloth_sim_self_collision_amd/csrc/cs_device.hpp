@@ -85,6 +85,7 @@ enum Flag : int {
   kSkip = 4,
   kTicketErr = 5,  // a reduction ticket was found nonzero after the solve
   kFlagNonFinite = 6,  // the step's displacement has an infinite or NaN entry
+  kSweepErr = 7,  // a strip of a sweep gave up waiting for another (never in a sound run)
   kNumFlag = 16
 };
 
@@ -191,6 +192,23 @@ struct DevCloth {
   double* f_dinv;  // D^-1 entry (r, j) the same way with v = j; v = 3: the forward sweep's right-hand side
   double* b_blk;
   int* ising;      // per-row singular-pivot flags of the last factorisation
+  // sweeps by strips (cs_strips.hip; st_nf == 0: the mesh does not fit them):
+  // strips, sub-levels and LDS ring of the two sweeps, records in the order
+  // they are read, import offsets, the row of each slot
+  int st_nf, st_nb, st_nsf, st_nsb, st_ring;
+  const int* st_fptr;
+  const int* st_bptr;
+  char* st_frec;
+  char* st_brec;
+  const int* st_fsrc;
+  const int* st_bsrc;
+  const int* st_frow;
+  const int* st_brow;
+  const int* st_fslot;  // forward slot of each row
+  int st_fstride;       // bytes of a forward record
+  int st_rhs_off;       // byte offset of lane 0's right-hand side in it
+  double* st_sb;        // forward result / backward right-hand side, 64 per sub-level
+  int* st_ticket;       // strips claimed; zero between launches
 };
 
 // Which cloth a block works on.  One: the cloth handed to the launch by value
@@ -202,6 +220,24 @@ struct DevCloth {
 // struct would keep a per-thread copy of a batch table entry in scratch memory.
 __device__ __forceinline__ double* pcg_dir(const DevCloth& c, int it) {
   return (it & 1) ? c.p[1] : c.p[0];
+}
+
+// A sweep result that is not there yet: a signalling NaN, which no arithmetic
+// instruction produces (they return quiet ones).
+__device__ __forceinline__ double unwritten() { return __hiloint2double(0x7ff4c107, 0); }
+__device__ __forceinline__ bool not_yet(double v) {
+  int hi = __double2hiint(v);
+  asm("" : "+v"(hi));  // a 32-bit compare (the compiler would widen it to 64)
+  return hi == 0x7ff4c107;
+}
+
+// entry e of the strip sweeps' right-hand side, and its result marked unwritten
+__device__ __forceinline__ void strip_put_rhs(const DevCloth& c, int e, double v) {
+  const int i = e / 3, slot = gptr(c.st_fslot)[i];
+  const size_t at = (size_t)(slot >> 3) * c.st_fstride + c.st_rhs_off +
+                    16 * ((slot & 7) * 8 + (e - 3 * i));
+  *(__attribute__((address_space(1))) double*)(c.st_frec + at) = v;
+  gptr(c.z)[e] = unwritten();
 }
 
 struct One {

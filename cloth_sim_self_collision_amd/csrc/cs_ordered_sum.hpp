@@ -439,6 +439,20 @@ __device__ inline double wave_walk(const double* buf, int len, double s,
   return s;
 }
 
+// One reduction: the addends, their count, the scratch and an optional flag
+// that cancels it.  A source policy Src provides
+//   __device__ SumJob job() const        -- the reduction of grid row blockIdx.y
+//   __device__ void finish(double) const -- consumes the exact sum (one thread)
+struct SumJob {
+  const double* t;
+  int n;
+  SumScratch w;
+  const int* skip;
+  // null, or a dot product: k_sum_tiles stores the addends x[i] * y[i] in t
+  const double* x;
+  const double* y;
+};
+
 // The chain over tiles b0 .. wend - 1 on one wave (every lane holds s):
 // tiles whose summary applies are added 64 per step, a failing tile is
 // walked from an LDS copy in buf.  code/tot/pmin/pmax hold the tiles'
@@ -493,32 +507,31 @@ __device__ __forceinline__ double chain_tiles(double s, int b0, int wend, const 
   return s;
 }
 
-// One reduction: the addends, their count, the scratch and an optional flag
-// that cancels it.  A source policy Src provides
-//   __device__ SumJob job() const        -- the reduction of grid row blockIdx.y
-//   __device__ void finish(double) const -- consumes the exact sum (one thread)
-struct SumJob {
-  const double* t;
-  int n;
-  SumScratch w;
-  const int* skip;
-};
-
-// approximate sum of every tile (any order); grid = (tiles of the largest job, jobs)
+// approximate sum of every tile (any order), and the addends of a dot product; grid = (tiles of the largest job, jobs)
 template <class Src>
 __global__ __launch_bounds__(kSumBlock) void k_sum_tiles(Src src) {
   const SumJob job = src.job();
   if (job.skip && *job.skip) return;
   if ((int)blockIdx.x >= sum_tiles(job.n)) return;
-  const double* __restrict__ t = job.t;
+  const double* t = job.t;
   const int n = job.n;
   __shared__ double wd[kSumWaves];
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const int base = blockIdx.x * kSumTile + tid * kSumPer;
   double a = 0.0;
+  if (job.x) {
 #pragma unroll
-  for (int j = 0; j < kSumPer; j++)
-    if (base + j < n) a += gload(t + base + j);
+    for (int j = 0; j < kSumPer; j++)
+      if (base + j < n) {
+        const double p = gload(job.x + base + j) * gload(job.y + base + j);
+        gstore(const_cast<double*>(t) + base + j, p);
+        a += p;
+      }
+  } else {
+#pragma unroll
+    for (int j = 0; j < kSumPer; j++)
+      if (base + j < n) a += gload(t + base + j);
+  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
   if (lane == 0) wd[wid] = a;

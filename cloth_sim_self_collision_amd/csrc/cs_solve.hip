@@ -438,18 +438,16 @@ __global__ __launch_bounds__(1024) void k_ilu_redo(Sel sel) {
   }
 }
 
-// forward then backward substitution, dst = (LU)^-1 src; optionally
-// prod = src .* dst for the next reduction (ilu_sparse.cpp:185-215, 295-324)
-// src == nullptr: the PCG operands (r in, z out, r.*z into prod)
+// forward then backward substitution, dst = (LU)^-1 src
+// (ilu_sparse.cpp:185-215, 295-324)
+// src == nullptr: the PCG operands (r in, z out)
 template <class Sel>
-__global__ __launch_bounds__(1024) void k_ilu_apply(Sel sel, const double* src, double* dst,
-                                                    double* prod) {
+__global__ __launch_bounds__(1024) void k_ilu_apply(Sel sel, const double* src, double* dst) {
   const DevCloth c = sel.cloth();
   if (c.flags[kSkip]) return;
   if (!src) {
     src = c.r;
     dst = c.z;
-    prod = c.prod;
   }
   for (int l = 0; l < c.nlf; l++) {
     const int b = c.lf_ptr[l], e = c.lf_ptr[l + 1];
@@ -490,8 +488,6 @@ __global__ __launch_bounds__(1024) void k_ilu_apply(Sel sel, const double* src, 
     }
     __syncthreads();
   }
-  if (prod)
-    for (int e = threadIdx.x; e < 3 * c.np; e += blockDim.x) prod[e] = src[e] * dst[e];
 }
 
 // ---------------------------------------------------------------------------
@@ -837,7 +833,7 @@ __device__ __forceinline__ void quad_sweep(const DevCloth& c, const Cuts& cuts, 
 
 // M^-1 (L+D)(I+D^-1 U) solve of the factor: forward sweep from the
 // right-hand side in forward-slot order (fwd_rhs_index) into c.sb, backward
-// sweep into dst (row order); prod = src_row .* dst when prod is given.
+// sweep into dst (row order).
 // One workgroup per connected component (blockIdx.x): the matrix is block
 // diagonal over them, so their sweeps are independent.
 // K: the packed blocks per row (DevCloth::kpack)
@@ -870,33 +866,17 @@ __device__ __forceinline__ void quad_component(const DevCloth& c, int comp, doub
   __syncthreads();
 }
 
+// dst == nullptr: the PCG's z
 template <int K, bool F32, class Sel>
-__global__ __launch_bounds__(kQuadThreads) void k_ilu_apply_quad(Sel sel, const double* src_row,
-                                                                 double* dst, double* prod) {
+__global__ __launch_bounds__(kQuadThreads) void k_ilu_apply_quad(Sel sel, double* dst) {
   const DevCloth c = sel.cloth();
   const int comp = blockIdx.x;
   if (c.flags[kSkip] || comp >= c.ncomp) return;  // batch grids fit the most components
-  if (!src_row) {
-    src_row = c.r;
-    dst = c.z;
-    prod = c.prod;
-  }
+  if (!dst) dst = c.z;
   __shared__ double ring[3][kRingLen];  // + the dummy and the zero entry
   __shared__ int cuts[kCutsLds + 1];
   if (threadIdx.x < 3) ring[threadIdx.x][kRingZero] = 0.0;  // never written again
   quad_component<K, F32>(c, comp, dst, ring, cuts);
-  if (!prod) return;
-  if (c.ncomp == 1) {
-    for (int e = threadIdx.x; e < 3 * c.np; e += blockDim.x)
-      gstore(prod + e, gload(src_row + e) * gload(dst + e));
-  } else {  // this component's rows: its forward slots
-    const int s0 = c.qf_ptr[c.qf_comp[comp]], s1 = c.qf_ptr[c.qf_comp[comp + 1]];
-    for (int k = threadIdx.x; k < 3 * (s1 - s0); k += blockDim.x) {
-      const int sl = s0 + k / 3;
-      const int e = 3 * gload(c.f_rci + 4 * sl) + (k - 3 * (k / 3));
-      gstore(prod + e, gload(src_row + e) * gload(dst + e));
-    }
-  }
 }
 
 // threads of a quad sweep: four per row of the widest sub-level (at most
@@ -907,29 +887,29 @@ inline int quad_threads(int qwidth) {
 }
 
 template <bool F32, class Sel>
-static void launch_quad_p(int kq, dim3 grid, dim3 tb, const Sel& sel, const double* src,
-                          double* dst, double* prod, hipStream_t s) {
+static void launch_quad_p(int kq, dim3 grid, dim3 tb, const Sel& sel, double* dst,
+                          hipStream_t s) {
   switch (kq) {
-    case 1: hipLaunchKernelGGL((k_ilu_apply_quad<1, F32, Sel>), grid, tb, 0, s, sel, src, dst, prod); break;
-    case 2: hipLaunchKernelGGL((k_ilu_apply_quad<2, F32, Sel>), grid, tb, 0, s, sel, src, dst, prod); break;
-    case 3: hipLaunchKernelGGL((k_ilu_apply_quad<3, F32, Sel>), grid, tb, 0, s, sel, src, dst, prod); break;
-    case 4: hipLaunchKernelGGL((k_ilu_apply_quad<4, F32, Sel>), grid, tb, 0, s, sel, src, dst, prod); break;
-    case 5: hipLaunchKernelGGL((k_ilu_apply_quad<5, F32, Sel>), grid, tb, 0, s, sel, src, dst, prod); break;
-    case 6: hipLaunchKernelGGL((k_ilu_apply_quad<6, F32, Sel>), grid, tb, 0, s, sel, src, dst, prod); break;
-    case 7: hipLaunchKernelGGL((k_ilu_apply_quad<7, F32, Sel>), grid, tb, 0, s, sel, src, dst, prod); break;
-    default: hipLaunchKernelGGL((k_ilu_apply_quad<8, F32, Sel>), grid, tb, 0, s, sel, src, dst, prod); break;
+    case 1: hipLaunchKernelGGL((k_ilu_apply_quad<1, F32, Sel>), grid, tb, 0, s, sel, dst); break;
+    case 2: hipLaunchKernelGGL((k_ilu_apply_quad<2, F32, Sel>), grid, tb, 0, s, sel, dst); break;
+    case 3: hipLaunchKernelGGL((k_ilu_apply_quad<3, F32, Sel>), grid, tb, 0, s, sel, dst); break;
+    case 4: hipLaunchKernelGGL((k_ilu_apply_quad<4, F32, Sel>), grid, tb, 0, s, sel, dst); break;
+    case 5: hipLaunchKernelGGL((k_ilu_apply_quad<5, F32, Sel>), grid, tb, 0, s, sel, dst); break;
+    case 6: hipLaunchKernelGGL((k_ilu_apply_quad<6, F32, Sel>), grid, tb, 0, s, sel, dst); break;
+    case 7: hipLaunchKernelGGL((k_ilu_apply_quad<7, F32, Sel>), grid, tb, 0, s, sel, dst); break;
+    default: hipLaunchKernelGGL((k_ilu_apply_quad<8, F32, Sel>), grid, tb, 0, s, sel, dst); break;
   }
 }
 
 // f32: the cloths' packed coefficients are FP32 (mixed precision)
 template <class Sel>
-static void launch_quad(int kq, bool f32, int qwidth, dim3 grid, const Sel& sel, const double* src,
-                        double* dst, double* prod, hipStream_t s) {
+static void launch_quad(int kq, bool f32, int qwidth, dim3 grid, const Sel& sel, double* dst,
+                        hipStream_t s) {
   const dim3 tb(quad_threads(qwidth));
   if (f32)
-    launch_quad_p<true>(kq, grid, tb, sel, src, dst, prod, s);
+    launch_quad_p<true>(kq, grid, tb, sel, dst, s);
   else
-    launch_quad_p<false>(kq, grid, tb, sel, src, dst, prod, s);
+    launch_quad_p<false>(kq, grid, tb, sel, dst, s);
 }
 
 bool sweep_shape(const DevCloth& c, int* waves, int* loads_fwd, int* loads_bwd) {
@@ -944,19 +924,26 @@ bool sweep_shape(const DevCloth& c, int* waves, int* loads_fwd, int* loads_bwd) 
   return true;
 }
 
-// one forward+backward substitution launch (variants give identical results):
-// 0 automatic (the quad sweep when the mesh allows it), 1 row-by-row CSR
-// sweep.  `rhs_ready`: the forward sweep's right-hand side already holds src
-// (the PCG producers write it).
-static void launch_sweep(const DevCloth& c, const double* src, double* dst, double* prod,
-                         hipStream_t s, bool rhs_ready = false) {
+// One forward+backward substitution launch (variants give identical results):
+// by strips where the mesh fits them (dst is then c.z), else in one workgroup
+// per component from the packed slots (the row-by-row CSR sweep for meshes
+// whose rows or ring do not fit those, and when it is selected).  Strips and
+// the one-workgroup sweep against each other, per launch: 256^2 sheet 391 and
+// 1263 us, 128^2 198 and 455 us, 32^2 52 and 74 us.
+// `rhs_ready`: the packed right-hand side already holds src (the PCG
+// producers write it).
+static void launch_sweep(const DevCloth& c, const double* src, double* dst, hipStream_t s,
+                         bool rhs_ready = false) {
   const One one{c, {}};
-  if (quad_ok(c) && c.sweep_variant != 1) {
+  if (strips_ok(c)) {
+    if (!rhs_ready) launch_strip_rhs(c, src, s);
+    launch_strip_sweep(c, s);
+  } else if (quad_ok(c) && c.sweep_variant != 1) {
     if (!rhs_ready)
       hipLaunchKernelGGL(k_gather_fslots<One>, dim3(grid_for(3L * c.np)), dim3(kTB), 0, s, one, src);
-    launch_quad(c.kpack, c.precision != 0, c.qwidth, dim3(c.ncomp), one, src, dst, prod, s);
+    launch_quad(c.kpack, c.precision != 0, c.qwidth, dim3(c.ncomp), one, dst, s);
   } else {
-    hipLaunchKernelGGL(k_ilu_apply<One>, dim3(1), dim3(1024), 0, s, one, src, dst, prod);
+    hipLaunchKernelGGL(k_ilu_apply<One>, dim3(1), dim3(1024), 0, s, one, src, dst);
   }
 }
 
@@ -1046,7 +1033,7 @@ __device__ __forceinline__ void spmv_dir_row(const DevCloth& c, int i, bool firs
   prod[3 * i + 2] = x2 * y2;
 }
 
-// p_new, A p_new and their products with a group of kSpG lanes per row: lane l forms block l's
+// p_new and A p_new with a group of kSpG lanes per row: lane l forms block l's
 // product (the diagonal block on lane deg), reading the row's contiguous
 // blocks side by side; the products are then added in the reference's order
 // (off-diagonal blocks in column order, the diagonal last) as spmv_dir_row
@@ -1116,39 +1103,45 @@ __global__ __launch_bounds__(kTB) void k_spmv_dir_g(Sel sel, int it) {
     x1 = z[3 * i + 1] + beta * pold[3 * i + 1];
     x2 = z[3 * i + 2] + beta * pold[3 * i + 2];
   }
-  const auto ap = gptr(c.ap), pnew = gptr(pcg_dir(c, it)), prod = gptr(c.prod);
+  const auto ap = gptr(c.ap), pnew = gptr(pcg_dir(c, it));
   ap[3 * i] = y0;
   ap[3 * i + 1] = y1;
   ap[3 * i + 2] = y2;
   pnew[3 * i] = x0;
   pnew[3 * i + 1] = x1;
   pnew[3 * i + 2] = x2;
-  prod[3 * i] = x0 * y0;
-  prod[3 * i + 1] = x1 * y1;
-  prod[3 * i + 2] = x2 * y2;
 }
 
-// one entry of k_update_rx: r -= alpha Ap, dx += alpha p, r .* r, and r as
-// the next forward sweep's right-hand side
-__device__ __forceinline__ void update_rx_elem(const DevCloth& c, int e, double alpha,
-                                               const double* __restrict__ p) {
+// where the next sweep reads its right-hand side
+enum RhsLayout : int { kRhsRows = 0, kRhsQuad = 1, kRhsStrips = 2 };
+
+__device__ __forceinline__ void put_rhs(const DevCloth& c, int e, double r, int layout) {
+  if (layout == kRhsStrips) {
+    strip_put_rhs(c, e, r);
+  } else if (layout == kRhsQuad) {
+    const int i = e / 3;
+    gptr(c.f_dinv)[fwd_rhs_index(c.np, gptr(c.fslot)[i], e - 3 * i)] = r;
+  }
+}
+
+// one entry of k_update_rx: r -= alpha Ap, dx += alpha p, and r as the next
+// forward sweep's right-hand side; returns r
+__device__ __forceinline__ double update_rx_elem(const DevCloth& c, int e, double alpha,
+                                                 const double* __restrict__ p, int layout) {
   const auto rr = gptr(c.r);
   const double r = rr[e] + -alpha * gptr(c.ap)[e];
   rr[e] = r;
   const auto dx = gptr(c.dx);
   dx[e] = dx[e] + alpha * gptr(p)[e];
-  gptr(c.prod2)[e] = r * r;
-  if (c.fslot) {
-    const int i = e / 3;
-    gptr(c.f_dinv)[fwd_rhs_index(c.np, gptr(c.fslot)[i], e - 3 * i)] = r;  // the next sweep's input
-  }
+  put_rhs(c, e, r, layout);
+  return r;
 }
 
-// r -= alpha A p; x += alpha p; prod = r .* r  (matrix_square_sparse.cpp:327-336)
+// r -= alpha A p; x += alpha p  (matrix_square_sparse.cpp:327-336)
 // Also snapshots kDone into kSkip for the kernels that run beside the next
 // convergence test (no kernel changes kDone while this one runs).
 template <class Sel>
-__global__ void k_update_rx(Sel sel, int it) {
+__global__ void k_update_rx(Sel sel, int it, int layout) {
   const DevCloth c = sel.cloth();
   const double* __restrict__ p = pcg_dir(c, it);
   const int done = c.flags[kDone];
@@ -1157,11 +1150,11 @@ __global__ void k_update_rx(Sel sel, int it) {
   if (done) return;
   const int e = e0 + (int)threadIdx.x;
   if (e >= 3 * c.np) return;
-  update_rx_elem(c, e, c.scal[kAlpha], p);
+  update_rx_elem(c, e, c.scal[kAlpha], p, layout);
 }
 
 template <class Sel>
-__global__ void k_pcg_init(Sel sel, double tol2) {
+__global__ void k_pcg_init(Sel sel, double tol2, int layout) {
   const DevCloth c = sel.cloth();
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e == 0) {
@@ -1171,6 +1164,7 @@ __global__ void k_pcg_init(Sel sel, double tol2) {
     c.flags[kSkip] = 0;
     c.flags[kTicketErr] = 0;
     c.flags[kFlagNonFinite] = 0;
+    c.flags[kSweepErr] = 0;
     c.scal[kTol2] = tol2;
     c.scal[kBeta] = 0.0;
   }
@@ -1178,11 +1172,7 @@ __global__ void k_pcg_init(Sel sel, double tol2) {
   const double b = c.b[e];
   c.r[e] = b;
   c.dx[e] = 0;
-  c.prod[e] = b * b;
-  if (c.fslot) {
-    const int i = e / 3;
-    c.f_dinv[fwd_rhs_index(c.np, c.fslot[i], e - 3 * i)] = b;
-  }
+  put_rhs(c, e, b, layout);
 }
 
 // ---------------------------------------------------------------------------
@@ -1192,32 +1182,37 @@ __global__ void k_pcg_init(Sel sel, double tol2) {
 // what the PCG does with a finished reduction (ilu_sparse.cpp:648-708)
 enum DotMode : int { kDotRr0 = 0, kDotRz0 = 1, kDotPap = 2, kDotRr = 3, kDotRz = 4, kDotFinal = 5 };
 
-// exact left-to-right sum of prod, then the PCG bookkeeping of `mode`
-// (ilu_sparse.cpp:646-700); every mode but the first is skipped once the
-// solve has converged.  The (r, z) reductions run beside the convergence test
-// that may set kDone, so they read its snapshot kSkip (k_update_rx), which is
-// constant while they run: every block of a launch takes the same branch.
+// exact left-to-right sum of a dot product's terms, then the PCG bookkeeping
+// of `mode` (ilu_sparse.cpp:646-700); every mode but the first is skipped once
+// the solve has converged.  The (r, z) reductions run beside the convergence
+// test that may set kDone, so they read its snapshot kSkip (k_update_rx),
+// which is constant while they run: every block of a launch takes the same
+// branch.
 //
-// Which products, scratch and skip flag a mode uses is decided on the host
-// (dot_src) and passed as two plain values, so job() is two two-way selects.
-// (A three-way choice of the skip pointer written as a conditional on `mode`
-// was compiled for gfx950 into a branch structure that left the addend and
-// skip-flag pointers undefined for the (p, Ap) mode, and the kernel faulted
-// on the load of the flag.)
-template <class Sel>
+// Which vectors a reduction multiplies is a template parameter, and which
+// scratch and skip flag it uses is decided on the host (launch_dot_of) and
+// passed as two plain values, so job() has two-way selects only.  (A
+// three-way choice of the skip pointer written as a conditional on `mode` was
+// compiled for gfx950 into a branch structure that left the addend and
+// skip-flag pointers undefined for the (p, Ap) mode, and the kernel faulted on
+// the load of the flag.)
+enum DotOf : int { kOfRr = 0, kOfRz = 1, kOfPap = 2 };
+
+template <class Sel, int kOf>
 struct DotSrc {
   Sel sel;
   int mode;
   int iter;
-  int aux;   // 1: the convergence test's products and scratch (prod2, sum2)
+  int aux;   // 1: the convergence test's addends and scratch (prod2, sum2)
   int skip;  // flag that cancels the reduction, -1: none
   __device__ SumJob job() const {
     const DevCloth c = sel.cloth();
-    const bool a = aux != 0;
-    // the convergence test reduces its own products with its own scratch: it
-    // runs beside the sweep and the (r, z) reduction
-    return SumJob{a ? c.prod2 : c.prod, 3 * c.np, a ? c.sum2 : c.sum,
-                  skip < 0 ? nullptr : c.flags + skip};
+    // the convergence test has its own: it runs beside the sweep and the
+    // (r, z) reduction
+    const double* x = kOf == kOfPap ? pcg_dir(c, iter) : c.r;
+    const double* y = kOf == kOfPap ? c.ap : kOf == kOfRz ? c.z : c.r;
+    return SumJob{aux != 0 ? c.prod2 : c.prod, 3 * c.np, aux != 0 ? c.sum2 : c.sum,
+                  skip < 0 ? nullptr : c.flags + skip, x, y};
   }
   __device__ void finish(double s) const {
     const DevCloth c = sel.cloth();
@@ -1261,24 +1256,23 @@ struct DotSrc {
   }
 };
 
-// the reduction of PCG mode `mode` (see DotSrc)
+// the reduction of PCG mode `mode` (see DotSrc) for `jobs` cloths of at most
+// max_np vertices
 template <class Sel>
-DotSrc<Sel> dot_src(const Sel& sel, int mode, int iter) {
+static void launch_dot_of(const Sel& sel, int mode, int iter, int max_np, int jobs,
+                          hipStream_t s) {
   const int aux = mode == kDotRr ? 1 : 0;
   const int skip = mode == kDotRr0 ? -1 : (mode == kDotRz0 || mode == kDotRz) ? kSkip : kDone;
-  return DotSrc<Sel>{sel, mode, iter, aux, skip};
+  if (mode == kDotPap)
+    launch_ordered_sum(DotSrc<Sel, kOfPap>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
+  else if (mode == kDotRz0 || mode == kDotRz)
+    launch_ordered_sum(DotSrc<Sel, kOfRz>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
+  else
+    launch_ordered_sum(DotSrc<Sel, kOfRr>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
 }
 
 static void launch_dot(const DevCloth& c, int mode, int iter, hipStream_t s) {
-  launch_ordered_sum(dot_src(One{c, {}}, mode, iter), 3 * c.np, 1, s);
-}
-
-template <class Sel>
-__global__ void k_square(Sel sel) {
-  const DevCloth c = sel.cloth();
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= 3 * c.np) return;
-  c.prod[e] = c.r[e] * c.r[e];
+  launch_dot_of(One{c, {}}, mode, iter, c.np, 1, s);
 }
 
 // after a solve every reduction has run to its end, which leaves its ticket
@@ -1288,7 +1282,8 @@ template <class Sel>
 __global__ void k_pcg_check(Sel sel) {
   const DevCloth c = sel.cloth();
   if (threadIdx.x == 0)
-    c.flags[kTicketErr] = (*c.sum.ticket != 0u || *c.sum2.ticket != 0u) ? 1 : 0;
+    c.flags[kTicketErr] =
+        (*c.sum.ticket != 0u || *c.sum2.ticket != 0u || c.flags[kSweepErr] != 0) ? 1 : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1350,7 +1345,10 @@ __global__ __launch_bounds__(kWgThreads) void k_pcg_wg(Sel sel, double tol2, int
     for (int i = tid; i < c.np; i += nth) spmv_dir_row(c, i, it == 0, beta, pold, pnew);
     __syncthreads();
     const double alpha = rz / wg_ordered_sum(c.prod, n3, ws);
-    for (int e = tid; e < n3; e += nth) update_rx_elem(c, e, alpha, pnew);
+    for (int e = tid; e < n3; e += nth) {
+      const double r = update_rx_elem(c, e, alpha, pnew, kRhsQuad);
+      gptr(c.prod2)[e] = r * r;
+    }
     __syncthreads();
     const double q = wg_ordered_sum(c.prod2, n3, ws) * inv_rr0;
     if (q < tol2) {
@@ -1478,7 +1476,14 @@ int launch_ilu(const DevCloth& c, hipStream_t s, Prof* prof) {
     hipLaunchKernelGGL(k_ilu_factor<One>, dim3(1), dim3(1024), 0, s, One{c, {}}, 0);
   hipLaunchKernelGGL(k_ilu_redo<One>, dim3(1), dim3(1024), 0, s, One{c, {}});
   CS_HIP(hipGetLastError());
-  return launch_pack_factor(c, s);
+  return kOk;
+}
+
+int ensure_packed(const DevCloth& c, bool strips, int* packed, hipStream_t s) {
+  const int want = strips ? kPackedStrips : kPackedQuad;
+  if (*packed & want) return kOk;
+  *packed |= want;
+  return strips ? launch_strip_pack(c, s) : launch_pack_factor(c, s);
 }
 
 int launch_pack_factor(const DevCloth& c, hipStream_t s) {
@@ -1496,8 +1501,10 @@ int launch_matvec(const DevCloth& c, double alpha, const double* x, double beta,
   return kOk;
 }
 
-int launch_ilu_apply(const DevCloth& c, const double* src, double* dst, hipStream_t s) {
-  launch_sweep(c, src, dst, nullptr, s);
+int launch_ilu_apply(const DevCloth& c, const double* src, double* dst, int* packed,
+                     hipStream_t s) {
+  if (int st = ensure_packed(c, strips_ok(c), packed, s)) return st;
+  launch_sweep(c, src, dst, s);
   CS_HIP(hipGetLastError());
   return kOk;
 }
@@ -1505,10 +1512,16 @@ int launch_ilu_apply(const DevCloth& c, const double* src, double* dst, hipStrea
 // Solve_PCG on the assembled system (c.b) with the factor in fdia/fcrs.
 // Result in c.dx; conv/iters in the device scalars.  `host_flags` is pinned
 // memory used to poll for convergence every `poll` iterations.
-int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, hipStream_t s, int poll,
-            Prof* prof, const PcgAux* aux) {
+int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, int* packed, hipStream_t s,
+            int poll, Prof* prof, const PcgAux* aux) {
   const long n3 = 3L * c.np;
   const bool wg = pcg_wg_ok(c) && c.pcg_variant == 2;
+  const bool strips = !wg && strips_ok(c);
+  const int layout = strips ? kRhsStrips : c.fslot ? kRhsQuad : kRhsRows;
+  {
+    ProfScope ps(prof, kProfOther);
+    if (int st = ensure_packed(c, strips, packed, s)) return st;
+  }
   if (wg) {
     ProfScope ps(prof, kProfPcgWg);
     launch_pcg_wg(c.kpack, dim3(1), One{c, {}}, tol * tol, maxit, s);
@@ -1517,7 +1530,8 @@ int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, hipStream
   }
   {
     ProfScope ps(prof, kProfOther);
-    hipLaunchKernelGGL(k_pcg_init<One>, dim3(grid_for(n3)), dim3(kTB), 0, s, One{c, {}}, tol * tol);
+    hipLaunchKernelGGL(k_pcg_init<One>, dim3(grid_for(n3)), dim3(kTB), 0, s, One{c, {}}, tol * tol,
+                       layout);
   }
   {
     ProfScope ps(prof, kProfReduce);
@@ -1525,7 +1539,7 @@ int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, hipStream
   }
   {
     ProfScope ps(prof, kProfSweep);
-    launch_sweep(c, c.r, c.z, c.prod, s, true);
+    launch_sweep(c, c.r, c.z, s, true);
   }
   {
     ProfScope ps(prof, kProfReduce);
@@ -1546,7 +1560,8 @@ int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, hipStream
     }
     {
       ProfScope ps(prof, kProfAxpy);
-      hipLaunchKernelGGL(k_update_rx<One>, dim3(grid_for(n3)), dim3(kTB), 0, s, One{c, {}}, it);
+      hipLaunchKernelGGL(k_update_rx<One>, dim3(grid_for(n3)), dim3(kTB), 0, s, One{c, {}}, it,
+                         layout);
     }
     if (aux) {
       // (r, r) and the convergence test beside the sweep; every later kernel
@@ -1565,7 +1580,7 @@ int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, hipStream
     }
     {
       ProfScope ps(prof, kProfSweep);
-      launch_sweep(c, c.r, c.z, c.prod, s, true);
+      launch_sweep(c, c.r, c.z, s, true);
     }
     {
       ProfScope ps(prof, kProfReduce);
@@ -1581,7 +1596,6 @@ int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, hipStream
   }
   if (!done) {
     // cap reached: report the achieved ratio (ilu_sparse.cpp:706-707)
-    hipLaunchKernelGGL(k_square<One>, dim3(grid_for(n3)), dim3(kTB), 0, s, One{c, {}});
     ProfScope ps(prof, kProfReduce);
     launch_dot(c, kDotFinal, maxit, s);
     CS_HIP(hipGetLastError());
@@ -1630,16 +1644,18 @@ __global__ void k_gather_done(const DevCloth* tab, int n, int* out) {
 
 static void launch_sweep_batch(const BatchView& b, hipStream_t s) {
   const Many m{b.tab, b.ptab};
-  if (b.piped) {
+  if (b.strips) {
+    launch_strip_sweep_batch(b, s);
+  } else if (b.piped) {
     // every cloth packed: r is already in slot order (k_pcg_init / k_update_rx)
-    launch_quad(b.kpack, b.f32, b.max_qwidth, dim3(b.max_ncomp, b.n), m, nullptr, nullptr, nullptr, s);
+    launch_quad(b.kpack, b.f32, b.max_qwidth, dim3(b.max_ncomp, b.n), m, nullptr, s);
   } else {
-    hipLaunchKernelGGL(k_ilu_apply<Many>, dim3(1, b.n), dim3(1024), 0, s, m, nullptr, nullptr, nullptr);
+    hipLaunchKernelGGL(k_ilu_apply<Many>, dim3(1, b.n), dim3(1024), 0, s, m, nullptr, nullptr);
   }
 }
 
 static void launch_dot_batch(const BatchView& b, int mode, int iter, hipStream_t s) {
-  launch_ordered_sum(dot_src(Many{b.tab, b.ptab}, mode, iter), 3 * b.max_np, b.n, s);
+  launch_dot_of(Many{b.tab, b.ptab}, mode, iter, b.max_np, b.n, s);
 }
 
 int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int* dgather,
@@ -1647,6 +1663,7 @@ int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int
   const Many m{b.tab, b.ptab};
   const int B = b.n;
   const unsigned gv = grid_for(3L * b.max_np), gp = grid_for(b.max_np);
+  const int layout = b.strips ? kRhsStrips : b.piped ? kRhsQuad : kRhsRows;
   {
     ProfScope ps(prof, kProfAssemble);
     hipLaunchKernelGGL(k_save_start<Many>, dim3(gv, B), dim3(kTB), 0, s, m);
@@ -1665,7 +1682,10 @@ int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int
     else
       hipLaunchKernelGGL(k_ilu_factor<Many>, dim3(1, B), dim3(1024), 0, s, m, 1);
     hipLaunchKernelGGL(k_ilu_redo<Many>, dim3(1, B), dim3(1024), 0, s, m);
-    hipLaunchKernelGGL(k_pack_factor<Many>, dim3(gp, B), dim3(kTB), 0, s, m);
+    if (b.strips && !b.wg)
+      launch_strip_pack_batch(b, s);
+    else
+      hipLaunchKernelGGL(k_pack_factor<Many>, dim3(gp, B), dim3(kTB), 0, s, m);
   }
   CS_HIP(hipGetLastError());
   if (b.wg) {
@@ -1680,7 +1700,7 @@ int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int
   }
   {
     ProfScope ps(prof, kProfOther);
-    hipLaunchKernelGGL(k_pcg_init<Many>, dim3(gv, B), dim3(kTB), 0, s, m, tol * tol);
+    hipLaunchKernelGGL(k_pcg_init<Many>, dim3(gv, B), dim3(kTB), 0, s, m, tol * tol, layout);
   }
   {
     ProfScope ps(prof, kProfReduce);
@@ -1709,7 +1729,7 @@ int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int
     {
       ProfScope ps(prof, kProfAxpy);
       hipLaunchKernelGGL(k_update_rx<ManyRows>, dim3(b.nvecblk), dim3(kTB), 0, s,
-                         ManyRows{b.tab, b.ptab, b.vecmap}, it);
+                         ManyRows{b.tab, b.ptab, b.vecmap}, it, layout);
     }
     if (aux) {
       // as in run_pcg: the convergence test of every cloth beside the sweep
@@ -1744,7 +1764,6 @@ int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int
   }
   if (!done) {
     // cloths at the cap report their achieved ratio; converged ones skip
-    hipLaunchKernelGGL(k_square<Many>, dim3(gv, B), dim3(kTB), 0, s, m);
     ProfScope ps(prof, kProfReduce);
     launch_dot_batch(b, kDotFinal, maxit, s);
   }

@@ -27,15 +27,35 @@ int launch_assemble(const DevCloth& c, const Params& P, hipStream_t s, Prof* pro
 int launch_ilu(const DevCloth& c, hipStream_t s, Prof* prof = nullptr);
 // rearrange the factor for the packed sweeps (after any change of fdia/fcrs)
 int launch_pack_factor(const DevCloth& c, hipStream_t s);
+// sweeps by strips (cs_strips.hip): one wave per strip of rows.  strips_ok:
+// the cloth's sweeps take them (the mesh fits and the row-by-row sweep is not
+// selected)
+bool strips_ok(const DevCloth& c);
+int strip_record_bytes(bool fwd, int K);
+int strip_rhs_offset(int K);
+// the records' metadata and the import offsets from device copies of the plan
+// (cs_strips.hpp: col and import of that sweep, slot of the backward one)
+int launch_strip_meta(const DevCloth& c, bool fwd, const unsigned short* col, const int* import,
+                      const int* bslot, hipStream_t s);
+int launch_strip_pack(const DevCloth& c, hipStream_t s);   // the factor into the records
+int launch_strip_reset(const DevCloth& c, hipStream_t s);  // before the first sweep, or after kSweepErr
+void launch_strip_rhs(const DevCloth& c, const double* x, hipStream_t s);
+void launch_strip_sweep(const DevCloth& c, hipStream_t s);
+// which packed copies of the factor are current (they are made when a solve
+// first needs them)
+enum Packed : int { kPackedQuad = 1, kPackedStrips = 2 };
+int ensure_packed(const DevCloth& c, bool strips, int* packed, hipStream_t s);
 int launch_matvec(const DevCloth& c, double alpha, const double* x, double beta, double* y,
                   hipStream_t s);
-int launch_ilu_apply(const DevCloth& c, const double* src, double* dst, hipStream_t s);
+// dst = (LU)^-1 src; with the strip sweeps dst must be c.z
+int launch_ilu_apply(const DevCloth& c, const double* src, double* dst, int* packed,
+                     hipStream_t s);
 // the one-workgroup PCG solve (k_pcg_wg) applies to this cloth
 bool pcg_wg_ok(const DevCloth& c);
 // Solve_PCG from dx = 0 with r = b; poll convergence every `poll` iterations
 // (the one-workgroup solve needs no poll)
-int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, hipStream_t s, int poll,
-            Prof* prof = nullptr, const PcgAux* aux = nullptr);
+int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, int* packed, hipStream_t s,
+            int poll, Prof* prof = nullptr, const PcgAux* aux = nullptr);
 // x[v] = rest[v] + off for the swept vertices
 int launch_apply_sweep(const DevCloth& c, const int* verts, int n, const double off[3],
                        hipStream_t s);
@@ -56,6 +76,8 @@ struct BatchView {
   int kpack;   // ... with this many packed blocks per row
   bool wg;     // every cloth takes the one-workgroup PCG solve (one workgroup per cloth)
   bool f32;    // every cloth's packed sweep coefficients are FP32 (mixed precision)
+  bool strips;  // every cloth's sweeps go by strips
+  int max_strips, max_ring, max_subs;  // most strips of a sweep, LDS ring sub-levels, sub-levels of both sweeps
   const int2* rowmap;  // the SpMV's blocks: (cloth, first row), kSpmvRows rows each
   int nrowblk;         // entries of rowmap
   const int2* vecmap;  // the vector update's blocks: (cloth, first of 3 np entries)
@@ -72,5 +94,7 @@ constexpr int kVecBlock = 256;
 int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int* dgather,
                         int* hgather, hipStream_t s, Prof* prof = nullptr,
                         const PcgAux* aux = nullptr);
+void launch_strip_sweep_batch(const BatchView& b, hipStream_t s);
+void launch_strip_pack_batch(const BatchView& b, hipStream_t s);
 
 }  // namespace cs

@@ -6,7 +6,9 @@
 //    offset past the LDS ring, a level order that breaks a dependency, a BVH
 //    child out of range, a gather source past the elements) must each be
 //    rejected;
-// 3. through the cache: a miss writes the file, a second lookup hits and
+// 3. the strip plan of the sweeps, when the mesh has one, passes its own
+//    validator, and a planted ring offset does not;
+// 4. through the cache: a miss writes the file, a second lookup hits and
 //    returns the same setup, a file with one flipped payload byte is
 //    rejected and rebuilt (a miss), and the rebuilt setup equals the fresh one.
 // Prints "ok" and exits 0 when every check holds.
@@ -16,6 +18,7 @@
 #include <vector>
 
 #include "cs_setup.hpp"
+#include "cs_strips.hpp"
 
 using cs::MeshSetup;
 
@@ -83,6 +86,22 @@ int main(int argc, char** argv) {
     p.apply(t);
     if (cs::validate_setup(t, np, nt, nq, tri.data(), quad.data()).empty())
       return fail(std::string("validate_setup accepts a planted mistake: ") + p.what);
+  }
+
+  // the strip plan reads every block from the entry its column row was
+  // written to; a planted offset or import is caught
+  cs::StripPlan strips;
+  cs::build_strips(s, strips);
+  if (strips.ok) {
+    err = cs::validate_strips(s, strips);
+    if (!err.empty()) return fail(err);
+    for (size_t q = 0; q < strips.fwd.col.size(); q++)
+      if (strips.fwd.col[q]) {
+        strips.fwd.col[q] ^= cs::kStripEntry;
+        break;
+      }
+    if (s.nnz > 0 && cs::validate_strips(s, strips).empty())
+      return fail("validate_strips accepts a wrong ring offset");
   }
 
   // the cache
