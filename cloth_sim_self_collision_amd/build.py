@@ -24,7 +24,8 @@ BUILD_DIR = os.path.join(HERE, "_build")
 SOURCES = ["cs_setup.cpp", "cs_setup_cache.cpp", "cs_strips.cpp", "cs_api.cpp", "cs_solve.hip",
            "cs_strips.hip", "cs_contact.hip",
            "cs_elements.hip", "cs_noalloc.hip"]
-HEADERS = ["cs_math.hpp", "cs_ordered_sum.hpp", "cs_setup.hpp", "cs_strips.hpp",
+HEADERS = ["cs_math.hpp", "cs_ordered_sum.hpp", "cs_item_sum.hpp",
+           "cs_setup.hpp", "cs_strips.hpp",
            "cs_device.hpp", "cs_solve.hpp", "cs_contact.hpp"]
 
 ARCH = os.environ.get("CLOTHSIM_ARCH", "gfx950")

@@ -276,16 +276,12 @@ int build(Cloth* c, const cs_mesh* m) {
   const size_t ntile = (size_t)sum_tiles(3 * np);
   A.reserve(&d.sum.tsum, ntile);
   A.reserve(&d.sum.code, ntile);
-  A.reserve(&d.sum.tot, ntile);
-  A.reserve(&d.sum.pmin, ntile);
-  A.reserve(&d.sum.pmax, ntile);
+  A.reserve(&d.sum.items, ntile * kItemCap);
   A.reserve(&d.sum.ticket, 1);
   A.reserve(&d.prod2, 3 * (size_t)np);
   A.reserve(&d.sum2.tsum, ntile);
   A.reserve(&d.sum2.code, ntile);
-  A.reserve(&d.sum2.tot, ntile);
-  A.reserve(&d.sum2.pmin, ntile);
-  A.reserve(&d.sum2.pmax, ntile);
+  A.reserve(&d.sum2.items, ntile * kItemCap);
   A.reserve(&d.sum2.ticket, 1);
   A.reserve(&c->sum_stats, kNumSumStat);
   A.reserve(&d.scal, kNumScal);

@@ -7,7 +7,7 @@
 #include <string>
 #include <vector>
 
-#include "cs_ordered_sum.hpp"
+#include "cs_item_sum.hpp"
 #include "cs_setup.hpp"
 
 namespace cs {

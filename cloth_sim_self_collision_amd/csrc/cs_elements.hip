@@ -8,7 +8,7 @@
 #include "../../include/clothsim.h"
 #include "cs_device.hpp"
 #include "cs_math.hpp"
-#include "cs_ordered_sum.hpp"
+#include "cs_item_sum.hpp"
 
 namespace cs {
 
@@ -218,11 +218,11 @@ extern "C" int cs_selftest_ordered_sum(int n, const double* t, double* out) {
   SumScratch w{};
   const int nt = sum_tiles(n);
   if (s.get(&dt, n) || s.get(&dout, 1) || s.get(&w.tsum, nt) || s.get(&w.code, nt) ||
-      s.get(&w.tot, nt) || s.get(&w.pmin, nt) || s.get(&w.pmax, nt) || s.get(&w.ticket, 1))
+      s.get(&w.items, (long)nt * kItemCap) || s.get(&w.ticket, 1))
     return kHipError;
   CS_HIP(hipMemset(w.ticket, 0, sizeof(unsigned int)));
   if (n) CS_HIP(hipMemcpy(dt, t, sizeof(double) * n, hipMemcpyHostToDevice));
-  launch_ordered_sum(SumStore{SumJob{dt, n, w, nullptr}, dout}, n, 1, 0);
+  launch_item_sum(SumStore{SumJob{dt, n, w, nullptr}, dout}, n, 1, 0);
   CS_HIP(hipGetLastError());
   CS_HIP(hipMemcpy(out, dout, sizeof(double), hipMemcpyDeviceToHost));
   return kOk;

@@ -123,6 +123,7 @@ struct SumScratch {
   long long* pmin;       // minimum inclusive integer prefix inside the tile
   long long* pmax;       // maximum inclusive integer prefix
   unsigned int* ticket;  // blocks finished; zero between launches
+  struct SumItem* items;  // cs_item_sum.hpp: items of every tile (code holds their count)
   // optional counters (null: off): sums, tiles, tiles applied in O(1),
   // walker steps, burst elements; device wall-clock ticks spent in the
   // chain, in the walker (bursts included) and in bursts
@@ -332,16 +333,16 @@ __device__ inline int wave_burst(const double* buf, int m, int len, double& s) {
   return k;
 }
 
-// Adds buf[0, len) (a tile, len <= kSumTile) onto s exactly and returns the
+// Adds buf[first, len) (of a tile, len <= kSumTile) onto s exactly and returns the
 // result; one wave, s the same in every lane.  Reads up to buf[kSumBuf - 1].
 __device__ inline double wave_walk(const double* buf, int len, double s,
-                                   unsigned long long* stats) {
+                                   unsigned long long* stats, int first = 0) {
   const int lane = threadIdx.x & 63;
   const double two52 = 4503599627370496.0;  // 2^52
   const double lo52 = two52 + 1.0, hi53 = 2.0 * two52 - 1.0;
   unsigned long long steps = 0, burst = 0, burst_ticks = 0;
   const unsigned long long walk_t0 = stats ? wall_clock64() : 0;
-  int pos = 0;
+  int pos = first;
   while (pos < len) {
     if (isnan(s)) break;  // NaN absorbs every later addend
     steps++;

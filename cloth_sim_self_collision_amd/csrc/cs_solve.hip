@@ -12,7 +12,7 @@
 
 #include "cs_device.hpp"
 #include "cs_math.hpp"
-#include "cs_ordered_sum.hpp"
+#include "cs_item_sum.hpp"
 #include "cs_solve.hpp"
 
 namespace cs {
@@ -1177,7 +1177,7 @@ __global__ void k_pcg_init(Sel sel, double tol2, int layout) {
 
 // ---------------------------------------------------------------------------
 // reductions: the reference sums left to right (matrix_square_sparse.cpp:313-323);
-// ordered_sum_exact (cs_ordered_sum.hpp) reproduces that loop bit for bit.
+// the item sums (cs_item_sum.hpp) reproduce that loop bit for bit.
 
 // what the PCG does with a finished reduction (ilu_sparse.cpp:648-708)
 enum DotMode : int { kDotRr0 = 0, kDotRz0 = 1, kDotPap = 2, kDotRr = 3, kDotRz = 4, kDotFinal = 5 };
@@ -1264,11 +1264,11 @@ static void launch_dot_of(const Sel& sel, int mode, int iter, int max_np, int jo
   const int aux = mode == kDotRr ? 1 : 0;
   const int skip = mode == kDotRr0 ? -1 : (mode == kDotRz0 || mode == kDotRz) ? kSkip : kDone;
   if (mode == kDotPap)
-    launch_ordered_sum(DotSrc<Sel, kOfPap>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
+    launch_item_sum(DotSrc<Sel, kOfPap>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
   else if (mode == kDotRz0 || mode == kDotRz)
-    launch_ordered_sum(DotSrc<Sel, kOfRz>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
+    launch_item_sum(DotSrc<Sel, kOfRz>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
   else
-    launch_ordered_sum(DotSrc<Sel, kOfRr>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
+    launch_item_sum(DotSrc<Sel, kOfRr>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
 }
 
 static void launch_dot(const DevCloth& c, int mode, int iter, hipStream_t s) {
