@@ -313,7 +313,9 @@ int build(Cloth* c, const cs_mesh* m) {
   StripPlan T;
   build_strips(S, T);
   // the records are addressed with 32-bit byte offsets inside a result array
-  if (24LL * np >= (1LL << 31) || 512LL * T.bwd.nsub >= (1LL << 31)) T.ok = false;
+  if (24LL * np >= (1LL << 31) || 512LL * T.bwd.nsub >= (1LL << 31) ||
+      72LL * nnz >= (1LL << 31))
+    T.ok = false;
   int *stfp, *stbp, *stfs, *stbs, *stfr, *stbr, *stsl;
   const size_t nsf = T.ok ? T.fwd.nsub + kStripTail : 0, nsb = T.ok ? T.bwd.nsub + kStripTail : 0;
   A.reserve(&stfp, T.fwd.ptr.size());
@@ -326,7 +328,9 @@ int build(Cloth* c, const cs_mesh* m) {
   A.reserve(&d.st_frec, strip_record_bytes(true, T.k) * nsf);
   A.reserve(&d.st_brec, strip_record_bytes(false, T.k) * nsb);
   A.reserve(&d.st_sb, 64 * nsb);
-  A.reserve(&d.st_ticket, 1);
+  A.reserve(&d.st_ticket, 2);
+  int* strows;
+  A.reserve(&strows, 8 * kStripRows * nsf);
   double* host_pd;
   A.reserve(&host_pd, 4 * (size_t)np);
   if (int st = A.commit(c->stream)) return st;
@@ -385,6 +389,7 @@ int build(Cloth* c, const cs_mesh* m) {
   d.ncomp = S.ncomp;
   d.qwidth = S.qwidth;
   hipStream_t s = c->stream;
+  bool strip_reset = false;
   if (T.ok) {
     d.st_nf = (int)T.fwd.ptr.size() - 1;
     d.st_nb = (int)T.bwd.ptr.size() - 1;
@@ -398,6 +403,7 @@ int build(Cloth* c, const cs_mesh* m) {
     d.st_frow = stfr;
     d.st_brow = stbr;
     d.st_fslot = stsl;
+    d.st_rows = strows;
     d.st_fstride = strip_record_bytes(true, T.k);
     d.st_rhs_off = strip_rhs_offset(T.k);
     if (int st = upload(stfp, T.fwd.ptr, s)) return st;
@@ -426,7 +432,7 @@ int build(Cloth* c, const cs_mesh* m) {
     }
     dev_free(tmp, s);
     if (st != kOk) return st;
-    if (int st = launch_strip_reset(d, s)) return st;
+    strip_reset = true;  // once the arrays it reads are uploaded
   }
   CS_HIP(hipMemsetAsync(d.sum.ticket, 0, sizeof(unsigned int), s));
   CS_HIP(hipMemsetAsync(d.sum2.ticket, 0, sizeof(unsigned int), s));
@@ -495,6 +501,8 @@ int build(Cloth* c, const cs_mesh* m) {
   CS_HIP(hipMemsetAsync(d.flags, 0, sizeof(int) * kNumFlag, s));
   CS_HIP(hipMemsetAsync(d.scal, 0, sizeof(double) * kNumScal, s));
   c->contact.host_pd_buf = host_pd;
+  if (strip_reset)
+    if (int st = launch_strip_reset(d, s)) return st;
   if (int st = launch_bend_setup(d, c->P, s)) return st;
   if (int st = contact_init(c->contact, S, d, s)) return st;
   CS_HIP(hipStreamSynchronize(s));
@@ -947,6 +955,7 @@ int cs_ilu_factor(cs_cloth* p, int* n_singular) {
   c->packed = 0;
   CS_HIP(hipMemcpyAsync(c->hflags, c->d.flags, sizeof(int) * kNumFlag, hipMemcpyDeviceToHost, c->stream));
   if (int st = sync(c)) return st;
+  if (int st = check_solve(c)) return st;
   if (n_singular) *n_singular = c->hflags[kNsing];
   return kOk;
 }
@@ -1245,6 +1254,7 @@ extern "C" int cs_batch_create(int n, cs_cloth* const* cloths, cs_batch** out) {
   BatchView& v = b->view;
   v.n = n;
   v.piped = true;
+  v.strip_factor = true;
   for (Cloth* c : b->cl) {
     if (c->P.pcg_tol != b->tol || c->P.pcg_maxit != b->maxit) {
       delete b;
@@ -1263,6 +1273,7 @@ extern "C" int cs_batch_create(int n, cs_cloth* const* cloths, cs_batch** out) {
                           ? -1
                           : std::max(v.max_fu_blocks, d.fu_blocks);
     v.piped = v.piped && quad_ok(d) && (v.kpack == 0 || v.kpack == d.kpack);
+    v.strip_factor = v.strip_factor && strip_factor_ok(d);
     v.max_strips = std::max(v.max_strips, std::max(d.st_nf, d.st_nb));
     v.max_ring = std::max(v.max_ring, d.st_ring);
     v.max_subs = std::max(v.max_subs, d.st_nsf + d.st_nsb);

@@ -208,7 +208,10 @@ struct DevCloth {
   int st_fstride;       // bytes of a forward record
   int st_rhs_off;       // byte offset of lane 0's right-hand side in it
   double* st_sb;        // forward result / backward right-hand side, 64 per sub-level
-  int* st_ticket;       // strips claimed; zero between launches
+  int* st_ticket;       // strips claimed by the sweep and by the factorisation; zero between launches
+  // factorisation by strips: {row (-1: none), rowptr, lower blocks, blocks, first
+  // update, updates, 0, 0} per forward slot
+  const int* st_rows;
 };
 
 // Which cloth a block works on.  One: the cloth handed to the launch by value

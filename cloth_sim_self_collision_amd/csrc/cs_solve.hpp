@@ -41,6 +41,9 @@ int launch_strip_pack(const DevCloth& c, hipStream_t s);   // the factor into th
 int launch_strip_reset(const DevCloth& c, hipStream_t s);  // before the first sweep, or after kSweepErr
 void launch_strip_rhs(const DevCloth& c, const double* x, hipStream_t s);
 void launch_strip_sweep(const DevCloth& c, hipStream_t s);
+// block ILU(0) of the assembled system by strips (the pivot flags included)
+void launch_strip_factor(const DevCloth& c, hipStream_t s);
+bool strip_factor_ok(const DevCloth& c);
 // which packed copies of the factor are current (they are made when a solve
 // first needs them)
 enum Packed : int { kPackedQuad = 1, kPackedStrips = 2 };
@@ -77,6 +80,7 @@ struct BatchView {
   bool wg;     // every cloth takes the one-workgroup PCG solve (one workgroup per cloth)
   bool f32;    // every cloth's packed sweep coefficients are FP32 (mixed precision)
   bool strips;  // every cloth's sweeps go by strips
+  bool strip_factor;  // every cloth is factorised by strips
   int max_strips, max_ring, max_subs;  // most strips of a sweep, LDS ring sub-levels, sub-levels of both sweeps
   const int2* rowmap;  // the SpMV's blocks: (cloth, first row), kSpmvRows rows each
   int nrowblk;         // entries of rowmap
@@ -96,5 +100,6 @@ int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int
                         const PcgAux* aux = nullptr);
 void launch_strip_sweep_batch(const BatchView& b, hipStream_t s);
 void launch_strip_pack_batch(const BatchView& b, hipStream_t s);
+void launch_strip_factor_batch(const BatchView& b, hipStream_t s);
 
 }  // namespace cs

@@ -458,14 +458,239 @@ __global__ void k_strip_meta(DevCloth c, int fwd, const unsigned short* col, con
 }
 
 // st_sb as the first launch expects it: unwritten where a row's result goes,
-// zero elsewhere; the ticket at zero
+// zero elsewhere; the tickets at zero; the rows of the slots
 __global__ void k_strip_reset(DevCloth c) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e == 0) *c.st_ticket = 0;
+  if (e == 0) {
+    c.st_ticket[0] = c.st_ticket[1] = 0;
+    c.flags[kSweepErr] = 0;
+  }
+  if (e < (c.st_nsf + kStripTail) * kStripRows) {
+    const int i = c.st_frow[e];
+    int* m = const_cast<int*>(c.st_rows) + 8 * e;
+    m[0] = i;
+    m[1] = i < 0 ? 0 : c.rowptr[i];
+    m[2] = i < 0 ? 0 : c.diaind[i] - c.rowptr[i];
+    m[3] = i < 0 ? 0 : c.rowptr[i + 1] - c.rowptr[i];
+    m[4] = i < 0 ? 0 : c.fu_ptr[i];
+    m[5] = i < 0 ? 0 : c.fu_ptr[i + 1] - c.fu_ptr[i];
+    m[6] = m[7] = 0;
+  }
   if (e >= (c.st_nsb + kStripTail) * 64) return;
   const int lane = e & 63;
   c.st_sb[e] =
       (lane & 7) < 3 && c.st_brow[(e >> 6) * kStripRows + (lane >> 3)] >= 0 ? unwritten() : 0.0;
+}
+
+// ---------------------------------------------------------------------------
+// Block ILU(0) by strips (ilu_sparse.cpp:387-401, 507-569), the strips of the
+// forward sweep: two waves per strip, sixteen lanes per row, the eight rows of
+// a sub-level at once.  A row's operations are ilu_row's (cs_solve.hip) in its
+// order, as in k_ilu_factor_staged: the updates that share a lower block L_ik
+// target distinct blocks and run at once, one per lane, with k ascending.
+//
+// The upper blocks of other rows are taken as they are finished, by the same
+// strip or by others: fcrs holds "not written yet" before (k_strip_unwritten),
+// each is stored with device scope, and the lane that needs one polls it.  (An
+// upper block is always a product with D^-1, so it is never the marker.)
+// Strips are claimed in order and wait only for strips claimed before; the two
+// waves of a strip, which wait for each other, are one workgroup.  What does
+// not depend on other rows (the row's place, its update list, its matrix
+// blocks) is loaded one or two sub-levels ahead.
+//
+// What bounds it: per sub-level a store and a load of device scope, the up to
+// eight dependent update rounds and the 3 x 3 inverse, about 5.5 us, times
+// the levels (one workgroup walking the levels: 19 us each at 256^2).
+constexpr int kFsLanes = 16;   // lanes per row
+constexpr int kFsLayers = 2;   // updates a lane keeps in registers
+constexpr int kFsBlocks = 2 * kMaxBlocksPerRow + 1;  // blocks of a row at most, the diagonal included
+constexpr int kFsVals = (9 * kFsBlocks + kFsLanes - 1) / kFsLanes;
+constexpr int kFsSlot = 9 * kFsBlocks + 2;  // doubles per row in LDS
+constexpr int kFsThreads = kStripRows * kFsLanes;
+
+// every off-diagonal block of the factor unwritten, no singular pivot seen
+template <class Sel>
+__global__ void k_strip_unwritten(Sel sel) {
+  const DevCloth c = sel.cloth();
+  const long n = 9L * c.nnz;
+  const long stride = (long)gridDim.x * blockDim.x;
+  const long e0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e0 == 0) c.flags[kNsing] = 0;
+  for (long e = e0; e < n; e += stride) gstore(c.fcrs + e, unwritten());
+  for (long e = e0; e < c.np; e += stride) gstore(c.ising + e, 0);
+}
+
+struct FsRow {  // a slot's row: where it is, its blocks and updates
+  int i, rb, low, deg, u0, nu;
+};
+struct FsUpdates {
+  int code[kFsLayers];  // lower block | target << 8, -1: none
+  unsigned at[kFsLayers];  // byte offset of the upper block used
+};
+
+__device__ __forceinline__ FsRow fs_row(const DevCloth& c, int slot) {
+  const auto p = (const __attribute__((address_space(1))) int4v*)c.st_rows + 2 * slot;
+  const int4v a = p[0], b = p[1];
+  return FsRow{a.x, a.y, a.z, a.w, b.x, b.y};
+}
+__device__ __forceinline__ void fs_updates(const DevCloth& c, const FsRow& r, int t,
+                                           FsUpdates& u) {
+#pragma unroll
+  for (int m = 0; m < kFsLayers; m++) {
+    const int e = t + m * kFsLanes;
+    const bool has = e < r.nu;
+    const int p = has ? r.u0 + e : 0;
+    const int code = gptr(c.fu_code)[p], kj = gptr(c.fu_kj)[p];
+    u.code[m] = has ? code : -1;
+    u.at[m] = has ? 72u * (unsigned)kj : kStripNone;
+  }
+}
+// the row's matrix blocks, then its diagonal block: value q on lane q % 16
+__device__ __forceinline__ void fs_matrix(const DevCloth& c, const FsRow& r, int t,
+                                          double (&v)[kFsVals]) {
+  const int n = 9 * r.deg;
+#pragma unroll
+  for (int m = 0; m < kFsVals; m++) {
+    const int q = t + m * kFsLanes;
+    double x = 0.0;
+    if (r.i >= 0 && q < n + 9)
+      x = q < n ? gptr(c.crs)[(size_t)r.rb * 9 + q] : gptr(c.dia)[(size_t)r.i * 9 + (q - n)];
+    v[m] = x;
+  }
+}
+__device__ __forceinline__ void fs_block(__amdgpu_buffer_rsrc_t f, unsigned at, double (&u)[9]) {
+#pragma unroll
+  for (int q = 0; q < 9; q++) u[q] = res_load(f, at == kStripNone ? at : at + 8 * q);
+}
+__device__ __forceinline__ bool fs_missing(const double (&u)[9]) {
+  bool w = false;
+#pragma unroll
+  for (int q = 0; q < 9; q++) w = w || not_yet(u[q]);
+  return w;
+}
+// A_ij -= L_ik U_kj on the row in LDS (diagonal block after the others)
+__device__ __forceinline__ void fs_apply(double* sl, int deg, int code, const double (&u)[9]) {
+  const double* l = sl + (code & 0xff) * 9;
+  const int tg = (code >> 8) & 0xff;
+  double* a = sl + (tg == kFuDiag ? deg : tg) * 9;
+#pragma unroll
+  for (int r = 0; r < 3; r++) {
+    const double l0 = l[r * 3 + 0], l1 = l[r * 3 + 1], l2 = l[r * 3 + 2];
+    a[r * 3 + 0] -= l0 * u[0] + l1 * u[3] + l2 * u[6];
+    a[r * 3 + 1] -= l0 * u[1] + l1 * u[4] + l2 * u[7];
+    a[r * 3 + 2] -= l0 * u[2] + l1 * u[5] + l2 * u[8];
+  }
+}
+
+template <class Sel>
+__global__ __launch_bounds__(kFsThreads) void k_strip_factor(Sel sel) {
+  const DevCloth c = sel.cloth();
+  __shared__ double stage[kStripRows * kFsSlot];
+  __shared__ int s_strip;
+  const int grp = threadIdx.x / kFsLanes, t = threadIdx.x % kFsLanes;
+  double* sl = stage + grp * kFsSlot;
+  const __amdgpu_buffer_rsrc_t f = res_of(c.fcrs, (unsigned)c.nnz * 72u);
+  if (threadIdx.x == 0)
+    s_strip = __hip_atomic_fetch_add(c.st_ticket + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const int strip = __builtin_amdgcn_readfirstlane(s_strip);
+  // every workgroup makes one claim; the last one resets
+  if (strip == (int)gridDim.x - 1 && threadIdx.x == 0) store_device(c.st_ticket + 1, 0);
+  if (strip >= c.st_nf) return;
+  const int first = c.st_fptr[strip], end = c.st_fptr[strip + 1];
+  int gave_up = 0;
+  FsRow r = fs_row(c, first * kStripRows + grp), rn = fs_row(c, (first + 1) * kStripRows + grp);
+  FsUpdates up;
+  double av[kFsVals];
+  fs_updates(c, r, t, up);
+  fs_matrix(c, r, t, av);
+  for (int sub = first; sub < end; sub++) {
+    double u[kFsLayers][9];
+#pragma unroll
+    for (int m = 0; m < kFsLayers; m++) fs_block(f, up.at[m], u[m]);
+    // ahead (past the strip's end: another strip's rows or the tail, unused)
+    const FsRow rnn = fs_row(c, (sub + 2) * kStripRows + grp);
+    FsUpdates upn;
+    double avn[kFsVals];
+    fs_updates(c, rn, t, upn);
+    fs_matrix(c, rn, t, avn);
+    const int nv = r.i >= 0 ? 9 * (r.deg + 1) : 0;
+#pragma unroll
+    for (int m = 0; m < kFsVals; m++)
+      if (t + m * kFsLanes < nv) sl[t + m * kFsLanes] = av[m];
+    int polls = 0;
+    while (!gave_up && __builtin_amdgcn_ballot_w64(fs_missing(u[0]) || fs_missing(u[1])) != 0ull) {
+      asm volatile("" ::: "memory");  // every poll loads again
+#pragma unroll
+      for (int m = 0; m < kFsLayers; m++)
+        if (fs_missing(u[m])) fs_block(f, up.at[m], u[m]);
+      gave_up = __builtin_amdgcn_readfirstlane(++polls >= kSpinMax);
+    }
+    wave_lds_sync();
+    for (int k = 0; k < r.low; k++) {
+#pragma unroll
+      for (int m = 0; m < kFsLayers; m++)
+        if (up.code[m] >= 0 && (up.code[m] & 0xff) == k) fs_apply(sl, r.deg, up.code[m], u[m]);
+      // updates beyond the registers
+      for (int e = t + kFsLayers * kFsLanes; e < r.nu; e += kFsLanes) {
+        const int cd = gptr(c.fu_code)[r.u0 + e];
+        if ((cd & 0xff) != k) continue;
+        double x[9];
+        int n = 0;
+        do {
+          asm volatile("" ::: "memory");
+          fs_block(f, 72u * (unsigned)gptr(c.fu_kj)[r.u0 + e], x);
+        } while (fs_missing(x) && ++n < kSpinMax);
+        if (n >= kSpinMax) store_device(c.flags + kSweepErr, 1);
+        fs_apply(sl, r.deg, cd, x);
+      }
+      wave_lds_sync();
+    }
+    double* d = sl + r.deg * 9;
+    if (t == 0 && r.i >= 0) {
+      const double det = +d[0] * d[4] * d[8] + d[3] * d[7] * d[2] + d[6] * d[1] * d[5] -
+                         d[0] * d[7] * d[5] - d[6] * d[4] * d[2] - d[3] * d[1] * d[8];
+      if (fabs(det) > 1.0e-30) {
+        const double id = 1.0 / det;
+        double w[9];
+        for (int q = 0; q < 9; q++) w[q] = d[q];
+        d[0] = id * (w[4] * w[8] - w[5] * w[7]);
+        d[1] = id * (w[2] * w[7] - w[1] * w[8]);
+        d[2] = id * (w[1] * w[5] - w[2] * w[4]);
+        d[3] = id * (w[5] * w[6] - w[3] * w[8]);
+        d[4] = id * (w[0] * w[8] - w[2] * w[6]);
+        d[5] = id * (w[2] * w[3] - w[0] * w[5]);
+        d[6] = id * (w[3] * w[7] - w[4] * w[6]);
+        d[7] = id * (w[1] * w[6] - w[0] * w[7]);
+        d[8] = id * (w[0] * w[4] - w[1] * w[3]);
+      } else {
+        gstore(c.ising + r.i, 1);
+        atomicAdd(&c.flags[kNsing], 1);
+      }
+    }
+    wave_lds_sync();
+    // upper blocks first (others wait for them): D^-1 U, one block row each
+    const int up_rows = r.i >= 0 ? 3 * (r.deg - r.low) : 0;
+    for (int q = t; q < up_rows; q += kFsLanes) {
+      const int b = q / 3, row = q - 3 * b;
+      const double* w = sl + (r.low + b) * 9;
+      const double d0 = d[row * 3], d1 = d[row * 3 + 1], d2 = d[row * 3 + 2];
+      const unsigned at = 72u * (unsigned)(r.rb + r.low + b) + 24u * row;
+      res_store(f, at, d0 * w[0] + d1 * w[3] + d2 * w[6]);
+      res_store(f, at + 8, d0 * w[1] + d1 * w[4] + d2 * w[7]);
+      res_store(f, at + 16, d0 * w[2] + d1 * w[5] + d2 * w[8]);
+    }
+    const int low = r.i >= 0 ? 9 * r.low : 0;
+    for (int q = t; q < low; q += kFsLanes) res_store(f, 72u * (unsigned)r.rb + 8u * q, sl[q]);
+    if (r.i >= 0 && t < 9) gstore(c.fdia + (size_t)r.i * 9 + t, d[t]);
+    wave_lds_sync();  // the slot is reused by the next row
+    r = rn;
+    rn = rnn;
+    up = upn;
+#pragma unroll
+    for (int m = 0; m < kFsVals; m++) av[m] = avn[m];
+  }
+  if (gave_up && (threadIdx.x & 63) == 0) store_device(c.flags + kSweepErr, 1);
 }
 
 // a single solve's right-hand side x (row order) into the records, z unwritten
@@ -516,6 +741,21 @@ void launch_strip_sweep_batch(const BatchView& b, hipStream_t s) {
     launch_k<false>(b.kpack, grid, lds, m, s);
 }
 
+bool strip_factor_ok(const DevCloth& c) { return c.st_nf > 0 && c.fu_blocks > 0; }
+
+void launch_strip_factor(const DevCloth& c, hipStream_t s) {
+  const unsigned fill = (unsigned)std::min<long>(2048, (9L * c.nnz + 255) / 256 + 1);
+  hipLaunchKernelGGL(k_strip_unwritten<One>, dim3(fill), dim3(256), 0, s, One{c, {}});
+  hipLaunchKernelGGL(k_strip_factor<One>, dim3(c.st_nf), dim3(kFsThreads), 0, s, One{c, {}});
+}
+
+void launch_strip_factor_batch(const BatchView& b, hipStream_t s) {
+  const Many m{b.tab, b.ptab};
+  const unsigned fill = (unsigned)std::min<long>(256, (9L * b.max_nnz + 255) / 256 + 1);
+  hipLaunchKernelGGL(k_strip_unwritten<Many>, dim3(fill, b.n), dim3(256), 0, s, m);
+  hipLaunchKernelGGL(k_strip_factor<Many>, dim3(b.max_strips, b.n), dim3(kFsThreads), 0, s, m);
+}
+
 int launch_strip_pack(const DevCloth& c, hipStream_t s) {
   const unsigned lanes = (unsigned)(c.st_nsf + c.st_nsb) * 64u;
   hipLaunchKernelGGL(k_strip_pack<One>, dim3((lanes + 255) / 256), dim3(256), 0, s, One{c, {}});
@@ -538,7 +778,7 @@ int launch_strip_meta(const DevCloth& c, bool fwd, const unsigned short* col, co
 }
 
 int launch_strip_reset(const DevCloth& c, hipStream_t s) {
-  const unsigned n = (unsigned)(c.st_nsb + kStripTail) * 64u;
+  const unsigned n = (unsigned)(std::max(c.st_nsf, c.st_nsb) + kStripTail) * 64u;
   hipLaunchKernelGGL(k_strip_reset, dim3((n + 255) / 256), dim3(256), 0, s, c);
   CS_HIP(hipGetLastError());
   return kOk;

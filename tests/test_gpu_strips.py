@@ -92,3 +92,22 @@ def test_solves_of_each_layout_alternate(sim_mod):
         strips = d.ilu_solve(b)
         d.set_option(1, 1)
         assert np.isfinite(strips).all() and np.array_equal(strips, d.ilu_solve(b))
+
+
+@pytest.mark.parametrize("name", sorted(MESHES))
+def test_factor_by_strips_bitwise(sim_mod, oracle_mod, name):
+    """The factorisation on the same meshes, on the assembled system and on a
+    random one (other update patterns of magnitude), twice each."""
+    cl = MESHES[name]()
+    o = oracle_mod.Oracle(cl, "port")
+    rng = np.random.default_rng(3)
+    with sim_mod.DeviceCloth(cl) as d:
+        dia, crs, b = d.assemble(cl.xyz, cl.uvw)
+        rdia = rng.standard_normal(dia.shape) + np.tile(9.0 * np.eye(3).reshape(-1), cl.np_)
+        rcrs = rng.standard_normal(crs.shape)
+        for A, B in ((dia, crs), (rdia, rcrs), (dia, crs)):
+            d.set_system(A, B, b)
+            assert d.ilu_factor() == 0
+            fd, fc = d.get_factor()
+            wd, wc = o.ilu(A, B)
+            assert np.array_equal(fd, wd) and np.array_equal(fc, wc)
