@@ -655,6 +655,7 @@ int cs_cloth_memory(const cs_cloth* p, long long* bytes) {
   // leaf pairs, two sort buffers, groups, the set, impulse links), sort
   // scratch and the per-vertex contact arrays
   *bytes = (long long)c->arena.bytes() + (long long)k.cap * 88 + (long long)k.tmp_bytes +
+           (long long)k.geom_cap * 128 +
            (long long)c->S.np * 64;
   return kOk;
 }

@@ -42,6 +42,8 @@ struct ContactState {
   int* vcount = nullptr;     // np + 1
   int* vstart = nullptr;     // np + 1
   int* vfill = nullptr;      // np + 1
+  void* geom = nullptr;      // proximity impulses: what depends on positions alone
+  int geom_cap = 0;
   // scalars
   int* counters = nullptr;   // device
   int* hcounters = nullptr;  // pinned mirror

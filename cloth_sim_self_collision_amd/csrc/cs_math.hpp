@@ -479,15 +479,21 @@ CS_HD bool fv_near(int i0, int i1, int i2, int i3, Vec3 p0, Vec3 p1, Vec3 p2, Ve
   return true;
 }
 
+// the edges' extents more than d apart along an axis (:421-426)
+CS_HD bool ee_apart(Vec3 p0, Vec3 p1, Vec3 q0, Vec3 q1, double d) {
+  if (q0.x + d < p0.x && q0.x + d < p1.x && q1.x + d < p0.x && q1.x + d < p1.x) return true;
+  if (q0.x - d > p0.x && q0.x - d > p1.x && q1.x - d > p0.x && q1.x - d > p1.x) return true;
+  if (q0.y + d < p0.y && q0.y + d < p1.y && q1.y + d < p0.y && q1.y + d < p1.y) return true;
+  if (q0.y - d > p0.y && q0.y - d > p1.y && q1.y - d > p0.y && q1.y - d > p1.y) return true;
+  if (q0.z + d < p0.z && q0.z + d < p1.z && q1.z + d < p0.z && q1.z + d < p1.z) return true;
+  if (q0.z - d > p0.z && q0.z - d > p1.z && q1.z - d > p0.z && q1.z - d > p1.z) return true;
+  return false;
+}
+
 // edge-edge proximity (:415-438)
 CS_HD bool ee_near(int i0, int i1, int j0, int j1, Vec3 p0, Vec3 p1, Vec3 q0, Vec3 q1, double d) {
   if (i0 == j0 || i0 == j1 || i1 == j0 || i1 == j1) return false;
-  if (q0.x + d < p0.x && q0.x + d < p1.x && q1.x + d < p0.x && q1.x + d < p1.x) return false;
-  if (q0.x - d > p0.x && q0.x - d > p1.x && q1.x - d > p0.x && q1.x - d > p1.x) return false;
-  if (q0.y + d < p0.y && q0.y + d < p1.y && q1.y + d < p0.y && q1.y + d < p1.y) return false;
-  if (q0.y - d > p0.y && q0.y - d > p1.y && q1.y - d > p0.y && q1.y - d > p1.y) return false;
-  if (q0.z + d < p0.z && q0.z + d < p1.z && q1.z + d < p0.z && q1.z + d < p1.z) return false;
-  if (q0.z - d > p0.z && q0.z - d > p1.z && q1.z - d > p0.z && q1.z - d > p1.z) return false;
+  if (ee_apart(p0, p1, q0, q1, d)) return false;
   double rp, rq;
   const double dist = edge_edge(p0, p1, q0, q1, rp, rq);
   if (dist > d) return false;
