@@ -689,10 +689,9 @@ __global__ void k_impulse_geom(const int* ce, int g, const double* X, double del
 
 // the velocity part of a proximity impulse: impulse_one's operations in its
 // order (its ccd == 0 branches)
-__device__ __forceinline__ void impulse_velocity(const ImpulseGeom* geom, double* U, double m) {
-  const ImpulseGeom o = *geom;
+__device__ __forceinline__ void impulse_velocity(const ImpulseGeom& o, Vec3 v0, Vec3 v1, Vec3 v2,
+                                                 Vec3 v3, double* U, double m) {
   if (o.kind == 0) return;
-  const Vec3 v0 = at(U, o.v[0]), v1 = at(U, o.v[1]), v2 = at(U, o.v[2]), v3 = at(U, o.v[3]);
   const Vec3 nrm = mk(o.n[0], o.n[1], o.n[2]);
   const double rel = o.kind == 1
                          ? dot(v3 - o.c[0] * v0 - o.c[1] * v1 - o.c[2] * v2, nrm)
@@ -763,6 +762,13 @@ __global__ void k_impulse_ready(int g, const int* pred, int* npred, int* ready, 
   if (c == 0) ready[atomicAdd(&counters[kReady], 1)] = i;
 }
 
+// a workgroup barrier that orders LDS only: loads and stores stay in flight
+__device__ __forceinline__ void lds_only_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Runs the ready contacts and every contact that becomes ready, round by
 // round, in one workgroup: a contact is ready once every earlier contact on
 // its vertices has run.  The contacts of a round share no vertex and each
@@ -771,60 +777,129 @@ __global__ void k_impulse_ready(int g, const int* pred, int* npred, int* ready, 
 // sweep.  Every contact enters a list once, so the loop ends after at most
 // g contacts; the count of those run goes to counters[kDoneCnt].
 //
-// A round's chain of memory latencies is what the schedule waits for, so
-// the lists after the first live in LDS (up to kDrainLds entries; the rest
-// of a longer round in the global list), and a contact releases its
-// successors before its impulse: they only run in the next round, after
-// the barrier that ends this one, and their counter atomics overlap the
-// impulse's loads.  lds_cap (at most kDrainLds) is the entries per LDS list;
-// a smaller value (the CLOTHSIM_DRAIN_LDS environment variable, a test hook)
-// sends more of every round through the global lists.
+// What bounds it: the chain of memory latencies of a round, times the rounds
+// (3122 for the 120 343 contacts of a folded 256^2 sheet).  So in proximity
+// passes half of the workgroup runs contacts and the other half fetches: a
+// running contact first releases its successors (they only run in the next
+// round, after the barrier that ends this one) and loads its velocities;
+// behind an LDS-only barrier the runners form and store the impulses while the
+// fetchers load the released contacts' geometry and successors, which come
+// from far memory, into LDS for the next round.  The four counter atomics of a
+// contact are all in flight together, at workgroup scope (no other workgroup
+// touches the counters).  Per round 2.2 us, from 3.6 with every contact
+// loading its own data: folded 256^2 sheet 6.8 ms from 11.4, 253 x 397 drop
+// 20 from 27, four stacked 128^2 sheets 6.4 from 7.4.
+// Released contacts are listed in LDS up to lds_cap, the rest of a longer round
+// in the global lists; the first kDrainRecs of a round have their data in LDS,
+// others load it themselves.  lds_cap (at most kDrainLds) is smaller only for
+// tests (the CLOTHSIM_DRAIN_LDS environment variable).
 constexpr int kDrainLds = 4096;
+constexpr int kDrainRun = 256;    // threads that run contacts, and as many that fetch
+constexpr int kDrainRecs = 256;   // contacts of a round whose data is in LDS
+constexpr int kDrainPieces = (int)sizeof(ImpulseGeom) / 16 + 1;  // 16 bytes each: geometry, successors
 
-__global__ __launch_bounds__(1024) void k_impulse_drain(const int* ce, const int* succ, int* npred,
-                                                        int* ready0, int* ready1, const double* X,
-                                                        double* U, double delta, double k,
-                                                        double dt, double m, int ccd,
-                                                        int* counters, int lds_cap,
-                                                        const ImpulseGeom* geom) {
-  __shared__ int n_next;
+__global__ __launch_bounds__(2 * kDrainRun) void k_impulse_drain(
+    const int* ce, const int* succ, int* npred, int* ready0, int* ready1, const double* X, double* U,
+    double delta, double k, double dt, double m, int ccd, int* counters, int lds_cap,
+    const ImpulseGeom* geom) {
+  __shared__ int count[2];  // contacts released for the next round, in turn
   __shared__ int lists[2][kDrainLds];
+  __shared__ int4 rec[2][kDrainRecs][kDrainPieces];
+  const int tid = threadIdx.x;
+  const bool runner = tid < kDrainRun;
   int n = counters[kReady];
   int *gcur = ready0, *gnxt = ready1;  // the first round's list and the spills
-  int cur = 0;                         // the LDS list of this round
+  int cur = 0;                         // the LDS list and data of this round
   bool first = true;                   // the first round reads k_impulse_ready's list
   int done = 0;
+  // data is fetched for contacts listed in LDS (a spilled entry is not visible
+  // behind the LDS-only barrier)
+  const int recs = min(kDrainRecs, lds_cap);
+  if (tid < 2) count[tid] = 0;
+  __syncthreads();
+  auto release = [&](int c) {
+    const int pos = atomicAdd(&count[cur ^ 1], 1);
+    if (pos < lds_cap)
+      lists[cur ^ 1][pos] = c;
+    else
+      gnxt[pos] = c;
+  };
+  // releases the successors of contact i; loads its velocities in between
+  auto begin = [&](int i, const int4& sc, const ImpulseGeom& o, Vec3 (&v)[4]) {
+    const int s4[4] = {sc.x, sc.y, sc.z, sc.w};
+    int left[4];
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+      // unconditional, so that the four are in flight together: without a
+      // successor the contact's own counter, which nothing reads any more
+      left[a] = __hip_atomic_fetch_sub(&npred[s4[a] >= 0 ? s4[a] : i], 1, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (geom)
+      for (int a = 0; a < 4; a++) v[a] = at(U, o.v[a]);
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+      if (s4[a] >= 0 && left[a] == 1) release(s4[a]);
+  };
+  auto finish = [&](int i, const ImpulseGeom& o, const Vec3 (&v)[4]) {
+    if (geom)
+      impulse_velocity(o, v[0], v[1], v[2], v[3], U, m);
+    else
+      impulse_one(ce + 5 * i, X, U, delta, k, dt, m, ccd);
+  };
   while (n > 0) {
-    if (threadIdx.x == 0) n_next = 0;
-    __syncthreads();
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
-      const int i = (first || t >= lds_cap) ? gcur[t] : lists[cur][t];
-      for (int a = 0; a < 4; a++) {
-        const int sc = succ[4 * i + a];
-        if (sc >= 0 && atomicSub(&npred[sc], 1) == 1) {
-          const int pos = atomicAdd(&n_next, 1);
-          if (pos < lds_cap)
-            lists[cur ^ 1][pos] = sc;
-          else
-            gnxt[pos] = sc;
-        }
+    ImpulseGeom o{};
+    Vec3 v[4];
+    int i = -1;
+    if (runner) {
+      // all but the last of this thread's contacts of a wide round
+      int t = tid;
+      for (; t + kDrainRun < n; t += kDrainRun) {
+        const int c = (first || t >= lds_cap) ? gcur[t] : lists[cur][t];
+        if (geom) o = geom[c];
+        begin(c, reinterpret_cast<const int4*>(succ)[c], o, v);
+        finish(c, o, v);
       }
-      if (geom)
-        impulse_velocity(geom + i, U, m);
-      else
-        impulse_one(ce + 5 * i, X, U, delta, k, dt, m, ccd);
+      if (t < n) {
+        i = (first || t >= lds_cap) ? gcur[t] : lists[cur][t];
+        int4 sc;
+        if (geom && !first && t < recs) {
+          int4 w[kDrainPieces];
+#pragma unroll
+          for (int p = 0; p < kDrainPieces; p++) w[p] = rec[cur][t][p];
+          __builtin_memcpy(&o, w, sizeof(o));
+          sc = w[kDrainPieces - 1];
+        } else {
+          if (geom) o = geom[i];
+          sc = reinterpret_cast<const int4*>(succ)[i];
+        }
+        begin(i, sc, o, v);
+      }
+    }
+    lds_only_barrier();  // the next round's list is complete; loads stay in flight
+    const int next = count[cur ^ 1];
+    if (runner) {
+      if (i >= 0) finish(i, o, v);
+      if (tid == 0) count[cur] = 0;  // read by every thread before the barrier above
+    } else if (geom) {
+      const int pieces = min(next, recs) * kDrainPieces;
+      for (int q = tid - kDrainRun; q < pieces; q += kDrainRun) {
+        const int e = q / kDrainPieces, p = q - e * kDrainPieces;
+        const int c = lists[cur ^ 1][e];
+        rec[cur ^ 1][e][p] = p < kDrainPieces - 1
+                                 ? reinterpret_cast<const int4*>(geom + c)[p]
+                                 : reinterpret_cast<const int4*>(succ)[c];
+      }
     }
     done += n;
-    __syncthreads();  // the round's velocities and the next list are complete
-    n = n_next;
+    __syncthreads();  // the round's velocities and the next round's data are complete
+    n = next;
     int* tmp = gcur;
     gcur = gnxt;
     gnxt = tmp;
     cur ^= 1;
     first = false;
-    __syncthreads();  // every thread has read n_next before it is reset
   }
-  if (threadIdx.x == 0) counters[kDoneCnt] = done;
+  if (tid == 0) counters[kDoneCnt] = done;
 }
 
 // ---------------------------------------------------------------------------
@@ -1232,7 +1307,7 @@ int impulses(ContactState& cs, const DevCloth& d, const Params& P, hipStream_t s
   }
   int lds_cap = kDrainLds;
   if (const char* e = getenv("CLOTHSIM_DRAIN_LDS")) lds_cap = std::min(std::max(atoi(e), 1), kDrainLds);
-  hipLaunchKernelGGL(k_impulse_drain, dim3(1), dim3(1024), 0, s, cs.ce, cs.succ, cs.npred,
+  hipLaunchKernelGGL(k_impulse_drain, dim3(1), dim3(2 * kDrainRun), 0, s, cs.ce, cs.succ, cs.npred,
                      cs.ready[0], cs.ready[1], X, U, P.clearance, P.k_contact, P.dt, P.mass, ccd,
                      cs.counters, lds_cap, ccd ? nullptr : (const ImpulseGeom*)cs.geom);
   CS_HIP(hipGetLastError());
