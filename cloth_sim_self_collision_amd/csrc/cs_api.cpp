@@ -142,7 +142,6 @@ struct Cloth {
   int* hflags = nullptr;  // pinned
   double* hscal = nullptr;
   int* ising = nullptr;   // per-row singular-pivot flags
-  PcgAux aux;             // convergence-test reduction beside the sweep
   unsigned long long* sum_stats = nullptr;  // reduction counters (while profiling)
   ContactState contact;
   bool have_x1 = false;
@@ -542,8 +541,7 @@ int internal_step(Cloth* c, double* conv, int* iters) {
   if (int st = launch_assemble(d, c->P, s, prof)) return st;
   if (int st = launch_ilu(d, s, prof)) return st;
   c->packed = 0;
-  if (int st = run_pcg(d, c->P.pcg_tol, c->P.pcg_maxit, c->hflags, &c->packed, s, c->poll, prof,
-                       &c->aux))
+  if (int st = run_pcg(d, c->P.pcg_tol, c->P.pcg_maxit, c->hflags, &c->packed, s, c->poll, prof))
     return st;
   if (int st = launch_finish_internal(d, c->P, s)) return st;
   CS_HIP(hipMemcpyAsync(c->hflags, d.flags, sizeof(int) * kNumFlag, hipMemcpyDeviceToHost, s));
@@ -596,9 +594,6 @@ int cs_cloth_create(const cs_mesh* mesh, const cs_params* params, cs_cloth** out
   c->P = to_params(params);
   int st = kOk;
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipStreamCreateWithFlags(&c->aux.stream, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&c->aux.updated, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&c->aux.tested, hipEventDisableTiming) != hipSuccess ||
       pinned_alloc((void**)&c->hflags, sizeof(int) * kNumFlag) != kOk ||
       pinned_alloc((void**)&c->hscal, sizeof(double) * kNumScal) != kOk) {
     set_error("stream or pinned buffer creation failed");
@@ -616,10 +611,9 @@ int cs_cloth_create(const cs_mesh* mesh, const cs_params* params, cs_cloth** out
 int cs_cloth_destroy(cs_cloth* p) {
   if (!p) return kOk;
   Cloth* c = H(p);
-  // every stream that used the cloth's memory is idle before it is released
+  // the stream that used the cloth's memory is idle before it is released
   // (the device memory after the work queued on the cloth's stream)
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  if (c->aux.stream) (void)hipStreamSynchronize(c->aux.stream);
   contact_release(c->contact, c->stream);
   c->prof.release();
   dev_free(c->sweep_verts, c->stream);
@@ -627,9 +621,6 @@ int cs_cloth_destroy(cs_cloth* p) {
   pinned_free(c->hflags);
   pinned_free(c->hscal);
   if (c->stream) (void)hipStreamDestroy(c->stream);
-  if (c->aux.stream) (void)hipStreamDestroy(c->aux.stream);
-  if (c->aux.updated) (void)hipEventDestroy(c->aux.updated);
-  if (c->aux.tested) (void)hipEventDestroy(c->aux.tested);
   delete c;
   return kOk;
 }
@@ -1015,7 +1006,7 @@ int cs_pcg_solve(cs_cloth* p, const double* b, double tol, int maxit, double* x,
   hipStream_t s = c->stream;
   const size_t n = sizeof(double) * 3 * c->S.np;
   CS_HIP(hipMemcpyAsync(c->d.b, b, n, hipMemcpyHostToDevice, s));
-  if (int st = run_pcg(c->d, tol, maxit, c->hflags, &c->packed, s, c->poll, nullptr, &c->aux))
+  if (int st = run_pcg(c->d, tol, maxit, c->hflags, &c->packed, s, c->poll))
     return st;
   if (x) CS_HIP(hipMemcpyAsync(x, c->d.dx, n, hipMemcpyDeviceToHost, s));
   if (r) CS_HIP(hipMemcpyAsync(r, c->d.r, n, hipMemcpyDeviceToHost, s));
@@ -1146,7 +1137,6 @@ struct Batch {
   int* dgather = nullptr;
   int* hgather = nullptr;  // pinned
   hipStream_t stream = nullptr;
-  PcgAux aux;  // convergence-test reductions beside the sweeps
   BatchView view{};
   double tol = 0.0;
   int maxit = 0;
@@ -1194,12 +1184,6 @@ Batch* HB(cs_batch* p) { return reinterpret_cast<Batch*>(p); }
 
 void batch_free(Batch* b) {
   if (b->stream) (void)hipStreamSynchronize(b->stream);
-  if (b->aux.stream) {
-    (void)hipStreamSynchronize(b->aux.stream);
-    (void)hipStreamDestroy(b->aux.stream);
-  }
-  if (b->aux.updated) (void)hipEventDestroy(b->aux.updated);
-  if (b->aux.tested) (void)hipEventDestroy(b->aux.tested);
   dev_free(b->dtab, b->stream);
   dev_free(b->ptab, b->stream);
   dev_free(b->rowmap, b->stream);
@@ -1285,9 +1269,6 @@ extern "C" int cs_batch_create(int n, cs_cloth* const* cloths, cs_batch** out) {
   b->htab.resize(n);
   b->hptab.resize(n);
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipStreamCreateWithFlags(&b->aux.stream, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&b->aux.updated, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&b->aux.tested, hipEventDisableTiming) != hipSuccess ||
       dev_alloc((void**)&b->dtab, sizeof(DevCloth) * n, b->stream) != kOk ||
       dev_alloc((void**)&b->ptab, sizeof(Params) * n, b->stream) != kOk ||
       dev_alloc((void**)&b->dgather, sizeof(int) * n, b->stream) != kOk ||
@@ -1383,7 +1364,7 @@ extern "C" int cs_batch_step(cs_batch* p, int nsteps, cs_step_stats* stats) {
       }
     for (Cloth* c : b->cl) c->packed = 0;  // the step makes new factors
     if (int st = batch_internal_step(b->view, b->tol, b->maxit, b->poll, b->dgather, b->hgather, s,
-                                     b->prof.on ? &b->prof : nullptr, &b->aux))
+                                     b->prof.on ? &b->prof : nullptr))
       return st;
     for (Cloth* c : b->cl) {
       c->packed = b->view.strips && !b->view.wg ? kPackedStrips : kPackedQuad;

@@ -69,7 +69,6 @@ enum Scal : int {
   kBeta = 3,
   kConv = 4,    // achieved residual ratio
   kTol2 = 5,    // tolerance squared
-  kLastDot = 6,
   kNumScal = 16
 };
 enum Flag : int {
@@ -77,11 +76,11 @@ enum Flag : int {
   kIters = 1,   // iteration count reported like Solve_PCG
   kNsing = 2,   // ILU pivots with |det| <= 1e-30
   kFirstSing11 = 3,  // row of the 11th singular pivot, np if none
-  // kDone as the main stream saw it before the convergence test of the
-  // iteration started beside the sweep: the sweep and the (r, z) reduction
-  // read this copy, which nothing changes while they run.  (A reduction whose
-  // blocks disagreed on a flag changing under them would leave its ticket
-  // short and corrupt every later reduction on the same scratch.)
+  // kDone as it was before the convergence test that runs beside the (r, z)
+  // reduction: the sweep and that reduction read this copy, which nothing
+  // changes while they run.  (A reduction whose blocks disagreed on a flag
+  // changing under them would leave its ticket short and corrupt every later
+  // reduction on the same scratch.)
   kSkip = 4,
   kTicketErr = 5,  // a reduction ticket was found nonzero after the solve
   kFlagNonFinite = 6,  // the step's displacement has an infinite or NaN entry
@@ -162,7 +161,7 @@ struct DevCloth {
   double* p[2];
   double* prod;  // element-wise products feeding the next reduction
   SumScratch sum;  // tile summaries of the ordered reductions over prod
-  double* prod2;   // r.*r of the convergence test, reduced on the auxiliary stream
+  double* prod2;   // r.*r of the convergence test, reduced beside (r, z)
   SumScratch sum2;
   double* scal;
   int* flags;
@@ -355,14 +354,6 @@ struct ProfScope {
   ~ProfScope() {
     if (p) p->end(id, s);
   }
-};
-
-// a second stream for the convergence-test reduction, which runs beside the
-// ILU sweep of the same PCG iteration (null: everything on one stream)
-struct PcgAux {
-  hipStream_t stream = nullptr;
-  hipEvent_t updated = nullptr;   // r and r.*r written
-  hipEvent_t tested = nullptr;    // (r, r) reduced and tested
 };
 
 struct Cloth;  // host handle (cs_api.cpp)

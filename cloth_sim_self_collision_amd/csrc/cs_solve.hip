@@ -1178,21 +1178,56 @@ __global__ void k_pcg_init(Sel sel, double tol2, int layout) {
 // reductions: the reference sums left to right (matrix_square_sparse.cpp:313-323);
 // the item sums (cs_item_sum.hpp) reproduce that loop bit for bit.
 
-// what the PCG does with a finished reduction (ilu_sparse.cpp:648-708)
+// What the PCG does with a finished reduction (ilu_sparse.cpp:648-708).
+// (r0, r0) before the loop, (r, z) before it, (p, Ap), (r, r) with the
+// convergence test, (r, z) in the loop, (r, r) at the iteration cap.
 enum DotMode : int { kDotRr0 = 0, kDotRz0 = 1, kDotPap = 2, kDotRr = 3, kDotRz = 4, kDotFinal = 5 };
 
-// exact left-to-right sum of a dot product's terms, then the PCG bookkeeping
-// of `mode` (ilu_sparse.cpp:646-700); every mode but the first is skipped once
-// the solve has converged.  The (r, z) reductions run beside the convergence
-// test that may set kDone, so they read its snapshot kSkip (k_update_rx),
-// which is constant while they run: every block of a launch takes the same
-// branch.
-//
-// Which vectors a reduction multiplies is a template parameter, and which
-// scratch and skip flag it uses is decided on the host (launch_dot_of) and
-// passed as two plain values, so job() has two-way selects only.  (A
-// three-way choice of the skip pointer written as a conditional on `mode` was
-// compiled for gfx950 into a branch structure that left the addend and
+__device__ __forceinline__ void dot_finish(const DevCloth& c, int mode, int iter, double s) {
+  switch (mode) {
+    case kDotRr0:
+      if (s < 1.0e-30) {
+        c.scal[kConv] = 0.0;
+        c.flags[kIters] = 0;
+        c.flags[kDone] = 1;
+        c.flags[kSkip] = 1;  // nothing runs beside this one
+      } else {
+        c.scal[kInvRr0] = 1.0 / s;
+      }
+      break;
+    case kDotRz0:
+      c.scal[kRz] = s;
+      break;
+    case kDotPap:
+      c.scal[kAlpha] = c.scal[kRz] / s;
+      break;
+    case kDotRr: {
+      const double q = s * c.scal[kInvRr0];
+      if (q < c.scal[kTol2]) {
+        c.scal[kConv] = sqrt(q);
+        c.flags[kIters] = iter;
+        c.flags[kDone] = 1;
+      }
+      break;
+    }
+    case kDotRz: {
+      c.scal[kBeta] = s / c.scal[kRz];
+      c.scal[kRz] = s;
+      break;
+    }
+    case kDotFinal:
+      c.scal[kConv] = sqrt(s * c.scal[kInvRr0]);
+      c.flags[kIters] = iter;
+      break;
+  }
+}
+
+// Exact left-to-right sum of a dot product's terms, then dot_finish.  Every
+// mode but the first is skipped once the solve has converged.  Which vectors a
+// reduction multiplies is a template parameter, and the skip flag is decided on
+// the host and passed as a plain value, so job() has two-way selects only.
+// (A three-way choice of the skip pointer written as a conditional on `mode`
+// was compiled for gfx950 into a branch structure that left the addend and
 // skip-flag pointers undefined for the (p, Ap) mode, and the kernel faulted on
 // the load of the flag.)
 enum DotOf : int { kOfRr = 0, kOfRz = 1, kOfPap = 2 };
@@ -1202,72 +1237,47 @@ struct DotSrc {
   Sel sel;
   int mode;
   int iter;
-  int aux;   // 1: the convergence test's addends and scratch (prod2, sum2)
   int skip;  // flag that cancels the reduction, -1: none
   __device__ SumJob job() const {
     const DevCloth c = sel.cloth();
-    // the convergence test has its own: it runs beside the sweep and the
-    // (r, z) reduction
     const double* x = kOf == kOfPap ? pcg_dir(c, iter) : c.r;
     const double* y = kOf == kOfPap ? c.ap : kOf == kOfRz ? c.z : c.r;
-    return SumJob{aux != 0 ? c.prod2 : c.prod, 3 * c.np, aux != 0 ? c.sum2 : c.sum,
-                  skip < 0 ? nullptr : c.flags + skip, x, y};
+    return SumJob{c.prod, 3 * c.np, c.sum, skip < 0 ? nullptr : c.flags + skip, x, y};
+  }
+  __device__ void finish(double s) const { dot_finish(sel.cloth(), mode, iter, s); }
+};
+
+// The two reductions after a sweep in one launch: (r, z) (blockIdx.z 0) and
+// the convergence test (r, r) (1), each with its own addends and scratch.  The
+// test may set kDone while the other runs, so (r, z) reads the snapshot kSkip
+// (k_update_rx), which is constant meanwhile: every block of a reduction takes
+// the same branch.
+template <class Sel>
+struct DotPairSrc {
+  Sel sel;
+  int iter;
+  __device__ SumJob job() const {
+    const DevCloth c = sel.cloth();
+    const bool rr = blockIdx.z != 0;
+    return SumJob{rr ? c.prod2 : c.prod, 3 * c.np, rr ? c.sum2 : c.sum,
+                  c.flags + (rr ? kDone : kSkip), c.r, rr ? c.r : c.z};
   }
   __device__ void finish(double s) const {
-    const DevCloth c = sel.cloth();
-    c.scal[kLastDot] = s;
-    switch (mode) {
-      case kDotRr0:
-        if (s < 1.0e-30) {
-          c.scal[kConv] = 0.0;
-          c.flags[kIters] = 0;
-          c.flags[kDone] = 1;
-          c.flags[kSkip] = 1;  // nothing runs beside this one
-        } else {
-          c.scal[kInvRr0] = 1.0 / s;
-        }
-        break;
-      case kDotRz0:
-        c.scal[kRz] = s;
-        break;
-      case kDotPap:
-        c.scal[kAlpha] = c.scal[kRz] / s;
-        break;
-      case kDotRr: {
-        const double q = s * c.scal[kInvRr0];
-        if (q < c.scal[kTol2]) {
-          c.scal[kConv] = sqrt(q);
-          c.flags[kIters] = iter;
-          c.flags[kDone] = 1;
-        }
-        break;
-      }
-      case kDotRz: {
-        c.scal[kBeta] = s / c.scal[kRz];
-        c.scal[kRz] = s;
-        break;
-      }
-      case kDotFinal:
-        c.scal[kConv] = sqrt(s * c.scal[kInvRr0]);
-        c.flags[kIters] = iter;
-        break;
-    }
+    dot_finish(sel.cloth(), blockIdx.z != 0 ? kDotRr : kDotRz, iter, s);
   }
 };
 
-// the reduction of PCG mode `mode` (see DotSrc) for `jobs` cloths of at most
-// max_np vertices
+// the reduction of PCG mode `mode` for `jobs` cloths of at most max_np vertices
 template <class Sel>
 static void launch_dot_of(const Sel& sel, int mode, int iter, int max_np, int jobs,
                           hipStream_t s) {
-  const int aux = mode == kDotRr ? 1 : 0;
-  const int skip = mode == kDotRr0 ? -1 : (mode == kDotRz0 || mode == kDotRz) ? kSkip : kDone;
+  const int skip = mode == kDotRr0 ? -1 : mode == kDotRz0 ? kSkip : kDone;
   if (mode == kDotPap)
-    launch_item_sum(DotSrc<Sel, kOfPap>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
-  else if (mode == kDotRz0 || mode == kDotRz)
-    launch_item_sum(DotSrc<Sel, kOfRz>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
+    launch_item_sum(DotSrc<Sel, kOfPap>{sel, mode, iter, skip}, 3 * max_np, jobs, s);
+  else if (mode == kDotRz0)
+    launch_item_sum(DotSrc<Sel, kOfRz>{sel, mode, iter, skip}, 3 * max_np, jobs, s);
   else
-    launch_item_sum(DotSrc<Sel, kOfRr>{sel, mode, iter, aux, skip}, 3 * max_np, jobs, s);
+    launch_item_sum(DotSrc<Sel, kOfRr>{sel, mode, iter, skip}, 3 * max_np, jobs, s);
 }
 
 static void launch_dot(const DevCloth& c, int mode, int iter, hipStream_t s) {
@@ -1519,7 +1529,7 @@ int launch_ilu_apply(const DevCloth& c, const double* src, double* dst, int* pac
 // Result in c.dx; conv/iters in the device scalars.  `host_flags` is pinned
 // memory used to poll for convergence every `poll` iterations.
 int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, int* packed, hipStream_t s,
-            int poll, Prof* prof, const PcgAux* aux) {
+            int poll, Prof* prof) {
   const long n3 = 3L * c.np;
   const bool wg = pcg_wg_ok(c) && c.pcg_variant == 2;
   const bool strips = !wg && strips_ok(c);
@@ -1569,30 +1579,16 @@ int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, int* pack
       hipLaunchKernelGGL(k_update_rx<One>, dim3(grid_for(n3)), dim3(kTB), 0, s, One{c, {}}, it,
                          layout);
     }
-    if (aux) {
-      // (r, r) and the convergence test beside the sweep; every later kernel
-      // of the solve checks the flag it sets, and x, r and the reported
-      // ratio and count do not depend on z
-      CS_HIP(hipEventRecord(aux->updated, s));
-      CS_HIP(hipStreamWaitEvent(aux->stream, aux->updated, 0));
-      {
-        ProfScope ps(prof, kProfReduce, aux->stream);
-        launch_dot(c, kDotRr, it, aux->stream);
-      }
-      CS_HIP(hipEventRecord(aux->tested, aux->stream));
-    } else {
-      ProfScope ps(prof, kProfReduce);
-      launch_dot(c, kDotRr, it, s);
-    }
     {
       ProfScope ps(prof, kProfSweep);
       launch_sweep(c, c.r, c.z, s, true);
     }
     {
+      // (r, z) and the convergence test together: x, r and the reported ratio
+      // and count do not depend on z, so the test may follow the sweep
       ProfScope ps(prof, kProfReduce);
-      launch_dot(c, kDotRz, it, s);
+      launch_item_sum(DotPairSrc<One>{One{c, {}}, it}, 3 * c.np, 1, s, 2);
     }
-    if (aux) CS_HIP(hipStreamWaitEvent(s, aux->tested, 0));
     CS_HIP(hipGetLastError());
     if ((it + 1) % poll == 0 || it + 1 == maxit) {
       CS_HIP(hipMemcpyAsync(host_flags, c.flags, sizeof(int) * kNumFlag, hipMemcpyDeviceToHost, s));
@@ -1665,7 +1661,7 @@ static void launch_dot_batch(const BatchView& b, int mode, int iter, hipStream_t
 }
 
 int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int* dgather,
-                        int* hgather, hipStream_t s, Prof* prof, const PcgAux* aux) {
+                        int* hgather, hipStream_t s, Prof* prof) {
   const Many m{b.tab, b.ptab};
   const int B = b.n;
   const unsigned gv = grid_for(3L * b.max_np), gp = grid_for(b.max_np);
@@ -1739,28 +1735,14 @@ int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int
       hipLaunchKernelGGL(k_update_rx<ManyRows>, dim3(b.nvecblk), dim3(kTB), 0, s,
                          ManyRows{b.tab, b.ptab, b.vecmap}, it, layout);
     }
-    if (aux) {
-      // as in run_pcg: the convergence test of every cloth beside the sweep
-      CS_HIP(hipEventRecord(aux->updated, s));
-      CS_HIP(hipStreamWaitEvent(aux->stream, aux->updated, 0));
-      {
-        ProfScope ps(prof, kProfReduce, aux->stream);
-        launch_dot_batch(b, kDotRr, it, aux->stream);
-      }
-      CS_HIP(hipEventRecord(aux->tested, aux->stream));
-    } else {
-      ProfScope ps(prof, kProfReduce);
-      launch_dot_batch(b, kDotRr, it, s);
-    }
     {
       ProfScope ps(prof, kProfSweep);
       launch_sweep_batch(b, s);
     }
     {
       ProfScope ps(prof, kProfReduce);
-      launch_dot_batch(b, kDotRz, it, s);
+      launch_item_sum(DotPairSrc<Many>{Many{b.tab, b.ptab}, it}, 3 * b.max_np, B, s, 2);
     }
-    if (aux) CS_HIP(hipStreamWaitEvent(s, aux->tested, 0));
     CS_HIP(hipGetLastError());
     if ((it + 1) % poll == 0 || it + 1 == maxit) {
       hipLaunchKernelGGL(k_gather_done, dim3(grid_for(B)), dim3(kTB), 0, s, b.tab, B, dgather);

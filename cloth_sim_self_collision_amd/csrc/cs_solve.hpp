@@ -58,7 +58,7 @@ bool pcg_wg_ok(const DevCloth& c);
 // Solve_PCG from dx = 0 with r = b; poll convergence every `poll` iterations
 // (the one-workgroup solve needs no poll)
 int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, int* packed, hipStream_t s,
-            int poll, Prof* prof = nullptr, const PcgAux* aux = nullptr);
+            int poll, Prof* prof = nullptr);
 // x[v] = rest[v] + off for the swept vertices
 int launch_apply_sweep(const DevCloth& c, const int* verts, int n, const double off[3],
                        hipStream_t s);
@@ -93,11 +93,9 @@ constexpr int kSpmvRows = 16;
 constexpr int kVecBlock = 256;
 // StepTime_InternalDynamicsILU for every cloth of the batch (start positions
 // saved, assembly, ILU(0), PCG, x += dx, v = dx/dt); dgather/hgather hold n
-// ints (device / pinned host) for the convergence poll; with aux, the (r, r)
-// reductions and tests run on aux->stream beside the sweeps
+// ints (device / pinned host) for the convergence poll
 int batch_internal_step(const BatchView& b, double tol, int maxit, int poll, int* dgather,
-                        int* hgather, hipStream_t s, Prof* prof = nullptr,
-                        const PcgAux* aux = nullptr);
+                        int* hgather, hipStream_t s, Prof* prof = nullptr);
 void launch_strip_sweep_batch(const BatchView& b, hipStream_t s);
 void launch_strip_pack_batch(const BatchView& b, hipStream_t s);
 void launch_strip_factor_batch(const BatchView& b, hipStream_t s);
