@@ -65,10 +65,10 @@ struct ItemShared {
 // Addend i of a job: t[i], or with kSelf and a dot product x[i] * y[i] formed
 // where it is needed.  Sums of at most kSelfTiles tiles take kSelf: every tile
 // adds up the tiles before it itself, which saves the launch of k_sum_tiles
-// (4 us and its gap; a tile's own work grows by up to seven tiles' reads): with
-// (r, z) and (r, r) also in one launch, a 32^2 drape's step went from 4.5 to 3.9
-// ms and a 61 x 96 drop's (18 tiles: two launches each) from 180 to 163 ms.
-constexpr int kSelfTiles = 8;
+// but costs the last tile about 2 us per tile before it.  Mean reduction of a
+// PCG, with and without: 14.3 / 17.1 us at 2 tiles, 16.3 / 17.8 at 3, 20.0 /
+// 18.5 at 5, 23.5 / 19.7 at 8, 40 / 25.6 at 18: the line lies between 3 and 5.
+constexpr int kSelfTiles = 4;
 template <bool kSelf>
 __device__ __forceinline__ double sum_term(const SumJob& job, int i) {
   if (kSelf && job.x) return gload(job.x + i) * gload(job.y + i);

@@ -56,7 +56,8 @@ KINDS = {"hover": _hover, "cancel": _cancel, "waves": _waves, "quiet": _mostly_q
 
 
 @pytest.mark.parametrize("kind", sorted(KINDS))
-@pytest.mark.parametrize("n", [1, 3, 1023, 1024, 1025, 4 * 1024 + 1, 63 * 1024 + 5, 64 * 1024,
+@pytest.mark.parametrize("n", [1, 3, 1023, 1024, 1025, 3 * 1024 + 7, 4 * 1024, 4 * 1024 + 1,
+                               63 * 1024 + 5, 64 * 1024,
                                65 * 1024 + 3, 200 * 1024 + 77])
 def test_items_equal_the_loop(sim_mod, kind, n):
     rng = np.random.default_rng(n)
