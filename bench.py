@@ -57,10 +57,10 @@ HBM_PEAK_GBS = 8000.0
 # scaled by what the counter reads for k_stream_copy of known size; the passes
 # and the scaling are in profiles/
 TRAFFIC_RATIO: dict = {
-    # profiles/fold256_hbm_traffic_pmc.md: (34065.4 * 2.000 + 4608.0) KiB / 59.98 MB
-    ("fold256", "ilu_sweep"): 1.242,
-    # profiles/served_stream_hbm_traffic_pmc.md: batched sweeps, 1.166 + 0.079
-    ("served", "ilu_sweep"): 1.245,
+    # profiles/fold256_hbm_traffic_pmc.md: (67342.1 * 2.000 + 7171.0) KiB / 59.98 MB
+    ("fold256", "ilu_sweep"): 2.422,
+    # profiles/served_stream_hbm_traffic_pmc.md: batched sweeps, 2.320 + 0.123
+    ("served", "ilu_sweep"): 2.443,
 }
 METRIC = "vertex-steps/s + p99 step latency, served vs plain GPU, at ≤1e-5 m pos err"
 
@@ -271,14 +271,12 @@ def serve_leg(args, copy_gbs) -> dict:
 
 def fold_leg(steps: int, copy_gbs, maxit: int) -> dict:
     """The single 256x256 folding cloth, plain step, with the ILU sweep's
-    launch time from HIP events on the cloth's stream, priced also against
-    two ceilings of its one-workgroup shape: one CU's read bandwidth
-    (cs_read_probe) and the issue time of the wave-load instructions one
-    launch issues (cs_sweep_shape x cs_issue_probe)."""
-    from cloth_sim_self_collision_amd.sim import DeviceCloth, issue_probe, read_probe
+    launch time from HIP events on the cloth's stream.  The sweep runs by
+    strips on many CUs, so the ceilings of a one-workgroup sweep (one CU's
+    read rate, its wave-load issue) do not apply to it and are not reported."""
+    from cloth_sim_self_collision_amd.sim import DeviceCloth
     cl = scene.fold_sweep(256, pcg_maxit=maxit)
     with DeviceCloth(cl) as d:
-        shape = d.sweep_shape()
         d.step(1)
         d.profile(True, sweep_only=True)
         lat, its = [], []
@@ -294,9 +292,6 @@ def fold_leg(steps: int, copy_gbs, maxit: int) -> dict:
         np_ = d.np_
     ach = b / (ms / n * 1e-3) / 1e9 if n else None
     avg_us = ms / n * 1e3 if n else None
-    one_cu = read_probe(1 << 23, 5, 1)
-    issue_ns = issue_probe(shape["waves"]) if shape["quad"] else None
-    floor_us = shape["wave_loads"] * issue_ns * 1e-3 if issue_ns else None
     print(f"[bench] fold256: {steps} steps in {wall:.2f} s", file=sys.stderr, flush=True)
     return {"workload": "fold256", "np": np_, "nt": cl.nt, "steps": steps,
             "vertex_steps_per_s": np_ * steps / wall, "ms_per_step": wall / steps * 1e3,
@@ -306,12 +301,7 @@ def fold_leg(steps: int, copy_gbs, maxit: int) -> dict:
                          "frac": ach / HBM_PEAK_GBS if ach else None, "bytes_per_launch": b,
                          "avg_launch_us": avg_us, "launches": n,
                          "traffic": TRAFFIC_RATIO[("fold256", "ilu_sweep")] * b,
-                         "frac_of_stream_copy": ach / copy_gbs if (ach and copy_gbs) else None,
-                         "one_cu_read_gbs": one_cu,
-                         "frac_of_one_cu_read": ach / one_cu if (ach and one_cu) else None,
-                         "sweep_shape": shape, "ns_per_wave_load": issue_ns,
-                         "issue_floor_us": floor_us,
-                         "frac_of_issue_floor": floor_us / avg_us if (floor_us and avg_us) else None}}
+                         "frac_of_stream_copy": ach / copy_gbs if (ach and copy_gbs) else None}}
 
 
 def stack_leg(steps: int, maxit: int) -> dict:

@@ -1,23 +1,25 @@
 // Contact-resolved velocity pass on the device
 // (self_collision_cloth.cpp:355-456, bvh_aabb.cpp).
 //
-//  refit      one launch, bottom-up: every leaf thread climbs while it is the
-//             second child to arrive (arrival counters are never reset: each
-//             refit adds exactly two arrivals per internal node, so the parity
-//             of the counter tells first from second).
-//  traverse   one thread per leaf walks the BVH in pre-order (stackless, the
-//             subtree end of every node is its skip link) and emits every
-//             later leaf whose box overlaps: exactly the leaf pairs the
-//             reference's recursion visits, oriented the same way (the leaf
-//             under the LCA's child 0 first).  The 6 face-vertex and 9
-//             edge-edge tests run on the pair in the reference's order.
+//  refit      the leaves, then one launch per tree depth, bottom-up.
+//  traverse   one wave walks the BVH in pre-order for a group of leaves
+//             (stackless, the subtree end of every node is its skip link) and
+//             lists every later leaf whose box overlaps: exactly the leaf
+//             pairs the reference's recursion visits, oriented the same way
+//             (the leaf under the LCA's child 0 first).
+//  narrow     the 6 face-vertex and 9 edge-edge tests of each pair, numbered
+//             in the reference's order: the tests that a pair needs are listed,
+//             then run one per thread, and a block's records are appended at
+//             one place.
 //  select     records are radix-sorted by canonical key; for a key found as
 //             both face-vertex and edge-edge the visit that comes first in the
 //             reference's depth-first order wins (std::set keeps the first
 //             insertion, bvh_aabb.h:96-102).
 //  impulses   Gauss-Seidel in key order, scheduled in rounds: a contact runs
 //             once every earlier contact sharing a vertex has run, so each
-//             velocity sees exactly the updates it sees sequentially.
+//             velocity sees exactly the updates it sees sequentially.  What
+//             does not depend on velocities (a proximity contact's distance
+//             and weights) is formed for all contacts at once before.
 //  zones      rigid impact zones by union-find in one workgroup, zone sums in
 //             ascending vertex order.
 #include <hip/hip_runtime.h>

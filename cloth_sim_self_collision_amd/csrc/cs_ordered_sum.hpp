@@ -1,7 +1,10 @@
 // Left-to-right floating-point summation, bit-identical to
 //     double s = 0.0; for (k = 0; k < n; k++) s += t[k];
 // (the reference's InnerProduct, matrix_square_sparse.cpp:313-325), computed
-// by two kernel launches over tiles of kSumTile elements.
+// by two kernel launches over tiles of kSumTile elements.  The PCG's launched
+// reductions cut the tiles further (cs_item_sum.hpp, built on this file); the
+// kernels here serve cs_ordered_sum_noalloc, and the walker and the chain the
+// solve that runs in one workgroup.
 //
 // Integer view of a binade.  Let s be a normal double with |s| in
 // [2^e, 2^(e+1)) and u = 2^(e-52) its ulp; s = S*u with the integer

@@ -5,9 +5,11 @@
 //
 // Bit-exactness: every value is produced by one thread in the reference's
 // operation order.  Assembly gathers each block's contributions in element
-// order (no atomics); the ILU factor and the triangular sweeps run one row
-// per thread over a precomputed level schedule; the PCG reductions are summed
-// left to right exactly as the reference's InnerProduct.
+// order (no atomics); the ILU factor and the triangular sweeps take the rows
+// in strips that wait for each other's rows (cs_strips.hip), or, where a mesh
+// does not fit those, by level of a precomputed schedule; the PCG reductions
+// are summed left to right exactly as the reference's InnerProduct
+// (cs_item_sum.hpp).
 #include <hip/hip_runtime.h>
 
 #include "cs_device.hpp"

@@ -184,18 +184,19 @@ int cs_batch_profile_read(cs_batch* b, int kind, double* total_ms, long long* la
 int cs_batch_step(cs_batch* b, int nsteps, cs_step_stats* stats);
 
 /* implementation choices (results are identical for every value):
- * CS_OPT_SWEEP: 0 automatic (the packed four-lanes-per-row sweep when
- *               the mesh allows it), 1 row-by-row CSR sweep
+ * CS_OPT_SWEEP: 0 automatic (the rows in strips, one wave each, when the mesh
+ *               allows it, else the packed four-lanes-per-row sweep of one
+ *               workgroup per component, else row by row), 1 row-by-row CSR
+ *               sweep
  * CS_OPT_PCG:   0 automatic (= 1), 1 one kernel launch per PCG operation
  *               with a host poll every 8 iterations, 2 the whole solve in one
  *               workgroup (one launch; needs the packed sweep and
  *               3 np <= 65536; a batch uses it for a step when all its cloths
  *               select it at that step,
  *               one workgroup per cloth, each iterating to its own
- *               convergence).  Measured: 2 is not faster than 1 for a 32^2
- *               cloth and slower for a 64-cloth batch of 24^2..128^2 cloths
- *               at the iteration cap (each cloth's SpMV and reductions then
- *               run on one CU) */
+ *               convergence).  2 keeps a cloth to one CU: slower than 1 for
+ *               a cloth alone or a batch of its own; for serving lanes of
+ *               small cloths that share the GPU with larger ones */
 /* CS_OPT_PRECISION: 0 FP64, bit-identical to the reference (default); 1
  *               mixed: the packed ILU sweep reads the factor's coefficients
  *               rounded to FP32 (D^-1, the vectors, SpMV, the reductions and
@@ -225,7 +226,7 @@ int cs_set_option(cs_cloth* c, int option, int value);
 int cs_profile_enable(cs_cloth* c, int on);
 int cs_profile_read(cs_cloth* c, int kind, double* total_ms, long long* launches);
 /* counters of the exact PCG reductions while profiling is on: out[8] =
- * reductions, tiles, tiles applied from their summary, binade-walker steps,
+ * reductions, tiles, tiles applied from their items, binade-walker steps,
  * elements added one by one, then nanoseconds (device wall clock, summed
  * over reductions) spent in the serial chain, in the binade walker (bursts
  * included) and in one-by-one bursts */
@@ -325,21 +326,23 @@ int cs_ordered_sum_noalloc(int n, const double* t, double* out, void* stream);
  * *gbs = 16 n reps / seconds / 1e9 (read + write) */
 int cs_bandwidth_probe(long long n, int reps, double* gbs);
 /* read-only streaming of n doubles by `blocks` workgroups of 512 threads
- * (blocks = 1: one CU, the ceiling of the one-workgroup ILU sweep), reps
+ * (blocks = 1: one CU, the ceiling of a one-workgroup ILU sweep), reps
  * times; n a multiple of 16384 * blocks; GB/s of reads */
 int cs_read_probe(long long n, int reps, int blocks, double* gbs);
 /* vector-load issue cost of one workgroup of `waves` waves (1..8) shaped like
- * the ILU sweep: each wave issues twelve 16-byte loads per step with two
+ * the one-workgroup ILU sweep: each wave issues twelve 16-byte loads per step with two
  * steps of loads in flight and an LDS-only barrier per step, quads of lanes
  * reading three consecutive 16-byte values (lane 3 repeats lane 2) from a
  * 64 MiB buffer; steps a multiple of 3.  *ns_per_load = time of one wave's
  * load instruction (the launch time over steps * waves * 12) */
 int cs_issue_probe(int waves, int steps, double* ns_per_load);
-/* shape of a cloth's ILU sweeps, for pricing them against cs_issue_probe:
+/* shape of a cloth's one-workgroup ILU sweeps (the one-workgroup solve's, and
+ * those of meshes the strips do not fit), for pricing them against
+ * cs_issue_probe:
  * out[8] = sub-levels of the longest component's forward and backward
  * sweeps, waves per sweep workgroup, vector loads per wave per forward and
- * per backward sub-level, components (one workgroup each), 1 if the packed
- * quad sweep is in use (0: the row-by-row sweep; the fields but the
+ * per backward sub-level, components (one workgroup each), 1 if the mesh and
+ * the options allow the packed quad sweep (0: the row-by-row sweep; the fields but the
  * components are then 0), and the wave-load instructions one launch issues in
  * its busiest workgroup (forward and backward; waves without a row in three
  * consecutive sub-levels skip their loads) */
