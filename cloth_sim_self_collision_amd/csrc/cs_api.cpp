@@ -516,12 +516,15 @@ int sync(Cloth* c) {
   return kOk;
 }
 
-// the flags of a finished solve (in c->hflags): its reductions and sweeps ended
-// as they must
+// The flags of a finished solve (in c->hflags): its reductions and sweeps ended
+// as they must.  After a wait that was given up the strips' markers are made as
+// a first launch expects them, before the return: the next solve may run on
+// another stream (a batch's).
 int check_solve(Cloth* c) {
   if (c->hflags[kSweepErr]) {
+    if (int st = launch_strip_reset(c->d, c->stream)) return st;
+    if (int st = sync(c)) return st;
     set_error("a strip of an ILU sweep gave up waiting for the strip before it");
-    (void)launch_strip_reset(c->d, c->stream);
     return kHipError;
   }
   if (c->hflags[kTicketErr]) {
@@ -1372,8 +1375,11 @@ extern "C" int cs_batch_step(cs_batch* p, int nsteps, cs_step_stats* stats) {
       CS_HIP(hipMemcpyAsync(c->hscal, c->d.scal, sizeof(double) * kNumScal, hipMemcpyDeviceToHost, s));
     }
     CS_HIP(hipStreamSynchronize(s));
-    for (size_t i = 0; i < n; i++)
-      if (int st = check_solve(b->cl[i])) return st;
+    // every member, so that each one's strips are reset where they failed
+    int solved = kOk;
+    for (Cloth* c : b->cl)
+      if (int st = check_solve(c); st != kOk && solved == kOk) solved = st;
+    if (solved != kOk) return solved;
     // contact passes: every cloth on its own stream, from up to
     // kContactThreads host threads (each pass waits on the host for its
     // contact counts, so passes of different cloths overlap those waits)

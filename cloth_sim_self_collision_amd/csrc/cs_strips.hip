@@ -50,6 +50,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdlib>
 
 #include "cs_device.hpp"
 #include "cs_solve.hpp"
@@ -129,6 +130,7 @@ struct Sweep {
   const int4v* src;            // import offsets, four sub-levels per entry
   __amdgpu_buffer_rsrc_t res;  // the array written and imported from
   __amdgpu_buffer_rsrc_t sbr;  // forward results (the backward right-hand side)
+  int polls;                   // of one wait before it is given up
 };
 
 template <class T>
@@ -219,8 +221,8 @@ __device__ __forceinline__ void set_wait(Set<K> (&q)[kSets], int n, const Sweep&
       if (!kFwd && not_yet(p.rhs))
         p.rhs = res_load(w.sbr, (unsigned)(sub + m) * 512u + threadIdx.x * 8);
     }
-  } while (waiting<kFwd>(q[n].imp, q[n].rhs) && ++polls < kSpinMax);
-  gave_up = __builtin_amdgcn_readfirstlane(polls >= kSpinMax);
+  } while (waiting<kFwd>(q[n].imp, q[n].rhs) && ++polls < w.polls);
+  gave_up = __builtin_amdgcn_readfirstlane(polls >= w.polls);
 }
 
 // the column rows' entries of a lane's blocks
@@ -349,7 +351,7 @@ __device__ __forceinline__ void strip_sweep(const Sweep& w, int first, int end, 
 
 template <int K, bool F32, class Sel>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void k_strip_sweep(Sel sel) {
+void k_strip_sweep(Sel sel, int polls) {
   const DevCloth c = sel.cloth();
   if (c.flags[kSkip]) return;
   extern __shared__ char lds[];
@@ -364,6 +366,7 @@ void k_strip_sweep(Sel sel) {
   b.rec = c.st_brec;
   b.src = reinterpret_cast<const int4v*>(c.st_bsrc);
   b.res = res_of(c.z, (unsigned)c.np * 24u);
+  f.polls = b.polls = polls;
   int gave_up = 0;
   while (true) {
     int t = 0;
@@ -583,7 +586,7 @@ __device__ __forceinline__ void fs_apply(double* sl, int deg, int code, const do
 }
 
 template <class Sel>
-__global__ __launch_bounds__(kFsThreads) void k_strip_factor(Sel sel) {
+__global__ __launch_bounds__(kFsThreads) void k_strip_factor(Sel sel, int polls_max) {
   const DevCloth c = sel.cloth();
   __shared__ double stage[kStripRows * kFsSlot];
   __shared__ int s_strip;
@@ -624,7 +627,7 @@ __global__ __launch_bounds__(kFsThreads) void k_strip_factor(Sel sel) {
 #pragma unroll
       for (int m = 0; m < kFsLayers; m++)
         if (fs_missing(u[m])) fs_block(f, up.at[m], u[m]);
-      gave_up = __builtin_amdgcn_readfirstlane(++polls >= kSpinMax);
+      gave_up = __builtin_amdgcn_readfirstlane(++polls >= polls_max);
     }
     wave_lds_sync();
     for (int k = 0; k < r.low; k++) {
@@ -640,8 +643,8 @@ __global__ __launch_bounds__(kFsThreads) void k_strip_factor(Sel sel) {
         do {
           asm volatile("" ::: "memory");
           fs_block(f, 72u * (unsigned)gptr(c.fu_kj)[r.u0 + e], x);
-        } while (fs_missing(x) && ++n < kSpinMax);
-        if (n >= kSpinMax) store_device(c.flags + kSweepErr, 1);
+        } while (fs_missing(x) && ++n < polls_max);
+        if (n >= polls_max) store_device(c.flags + kSweepErr, 1);
         fs_apply(sl, r.deg, cd, x);
       }
       wave_lds_sync();
@@ -704,21 +707,29 @@ __global__ void k_strip_rhs(DevCloth c, const double* x) {
 
 bool strips_ok(const DevCloth& c) { return c.st_nf > 0 && c.sweep_variant != 1; }
 
+// polls of one wait: kSpinMax, or fewer (0: every wait is given up) for tests
+// of what follows a wait that was given up (CLOTHSIM_STRIP_POLLS)
+static int wait_polls() {
+  const char* e = getenv("CLOTHSIM_STRIP_POLLS");
+  return e ? std::min(std::max(atoi(e), 0), kSpinMax) : kSpinMax;
+}
+
 int strip_record_bytes(bool fwd, int K) { return strip_pieces(fwd, K) * kPiece; }
 int strip_rhs_offset(int K) { return (strip_pairs(K) + 2) * kPiece + 8; }
 
 template <bool F32, class Sel>
 static void launch_k(int k, dim3 grid, size_t lds, const Sel& sel, hipStream_t s) {
   const dim3 tb(64);
+  const int polls = wait_polls();
   switch (k) {
-    case 1: hipLaunchKernelGGL((k_strip_sweep<1, F32, Sel>), grid, tb, lds, s, sel); break;
-    case 2: hipLaunchKernelGGL((k_strip_sweep<2, F32, Sel>), grid, tb, lds, s, sel); break;
-    case 3: hipLaunchKernelGGL((k_strip_sweep<3, F32, Sel>), grid, tb, lds, s, sel); break;
-    case 4: hipLaunchKernelGGL((k_strip_sweep<4, F32, Sel>), grid, tb, lds, s, sel); break;
-    case 5: hipLaunchKernelGGL((k_strip_sweep<5, F32, Sel>), grid, tb, lds, s, sel); break;
-    case 6: hipLaunchKernelGGL((k_strip_sweep<6, F32, Sel>), grid, tb, lds, s, sel); break;
-    case 7: hipLaunchKernelGGL((k_strip_sweep<7, F32, Sel>), grid, tb, lds, s, sel); break;
-    default: hipLaunchKernelGGL((k_strip_sweep<8, F32, Sel>), grid, tb, lds, s, sel); break;
+    case 1: hipLaunchKernelGGL((k_strip_sweep<1, F32, Sel>), grid, tb, lds, s, sel, polls); break;
+    case 2: hipLaunchKernelGGL((k_strip_sweep<2, F32, Sel>), grid, tb, lds, s, sel, polls); break;
+    case 3: hipLaunchKernelGGL((k_strip_sweep<3, F32, Sel>), grid, tb, lds, s, sel, polls); break;
+    case 4: hipLaunchKernelGGL((k_strip_sweep<4, F32, Sel>), grid, tb, lds, s, sel, polls); break;
+    case 5: hipLaunchKernelGGL((k_strip_sweep<5, F32, Sel>), grid, tb, lds, s, sel, polls); break;
+    case 6: hipLaunchKernelGGL((k_strip_sweep<6, F32, Sel>), grid, tb, lds, s, sel, polls); break;
+    case 7: hipLaunchKernelGGL((k_strip_sweep<7, F32, Sel>), grid, tb, lds, s, sel, polls); break;
+    default: hipLaunchKernelGGL((k_strip_sweep<8, F32, Sel>), grid, tb, lds, s, sel, polls); break;
   }
 }
 
@@ -746,14 +757,16 @@ bool strip_factor_ok(const DevCloth& c) { return c.st_nf > 0 && c.fu_blocks > 0;
 void launch_strip_factor(const DevCloth& c, hipStream_t s) {
   const unsigned fill = (unsigned)std::min<long>(2048, (9L * c.nnz + 255) / 256 + 1);
   hipLaunchKernelGGL(k_strip_unwritten<One>, dim3(fill), dim3(256), 0, s, One{c, {}});
-  hipLaunchKernelGGL(k_strip_factor<One>, dim3(c.st_nf), dim3(kFsThreads), 0, s, One{c, {}});
+  hipLaunchKernelGGL(k_strip_factor<One>, dim3(c.st_nf), dim3(kFsThreads), 0, s, One{c, {}},
+                     wait_polls());
 }
 
 void launch_strip_factor_batch(const BatchView& b, hipStream_t s) {
   const Many m{b.tab, b.ptab};
   const unsigned fill = (unsigned)std::min<long>(256, (9L * b.max_nnz + 255) / 256 + 1);
   hipLaunchKernelGGL(k_strip_unwritten<Many>, dim3(fill, b.n), dim3(256), 0, s, m);
-  hipLaunchKernelGGL(k_strip_factor<Many>, dim3(b.max_strips, b.n), dim3(kFsThreads), 0, s, m);
+  hipLaunchKernelGGL(k_strip_factor<Many>, dim3(b.max_strips, b.n), dim3(kFsThreads), 0, s, m,
+                     wait_polls());
 }
 
 int launch_strip_pack(const DevCloth& c, hipStream_t s) {

@@ -111,3 +111,54 @@ def test_factor_by_strips_bitwise(sim_mod, oracle_mod, name):
             fd, fc = d.get_factor()
             wd, wc = o.ilu(A, B)
             assert np.array_equal(fd, wd) and np.array_equal(fc, wc)
+
+
+def _states(devs):
+    return [a for d in devs for a in d.get_state()]
+
+
+def test_batch_steps_after_given_up_waits(sim_mod, monkeypatch):
+    """A step whose waits are given up is an error; every member's strips are
+    reset, so that the next step gives what it gives on new cloths."""
+    from cloth_sim_self_collision_amd import _lib
+    cls = [_grid(24, 24), _grid(33, 40), _grid(40, 24)]
+    for c in cls:
+        c.pcg_maxit = 40
+    runs = []
+    for fail in (False, True):
+        devs = [sim_mod.DeviceCloth(c) for c in cls]
+        try:
+            with sim_mod.DeviceBatch(devs) as b:
+                if fail:
+                    monkeypatch.setenv("CLOTHSIM_STRIP_POLLS", "0")
+                    with pytest.raises(_lib.ClothSimError, match="gave up waiting"):
+                        b.step(1)
+                    monkeypatch.delenv("CLOTHSIM_STRIP_POLLS")
+                    for d, c in zip(devs, cls):
+                        d.set_state(c.xyz, c.uvw)
+                        d.time = 0.0
+                b.step(2)
+                runs.append(_states(devs))
+        finally:
+            for d in devs:
+                d.close()
+    assert all(np.array_equal(g, w) for g, w in zip(*runs))
+
+
+def test_one_cloth_steps_after_given_up_waits(sim_mod, monkeypatch):
+    from cloth_sim_self_collision_amd import _lib
+    cl = _grid(33, 40)
+    cl.pcg_maxit = 40
+    with sim_mod.DeviceCloth(cl) as d:
+        d.step(2)
+        want = _states([d])
+    with sim_mod.DeviceCloth(cl) as d:
+        monkeypatch.setenv("CLOTHSIM_STRIP_POLLS", "0")
+        for call in (lambda: d.step(1), d.ilu_factor, lambda: d.ilu_solve(cl.xyz)):
+            with pytest.raises(_lib.ClothSimError, match="gave up waiting"):
+                call()
+        monkeypatch.delenv("CLOTHSIM_STRIP_POLLS")
+        d.set_state(cl.xyz, cl.uvw)
+        d.step(2)
+        got = _states([d])
+    assert all(np.array_equal(g, w) for g, w in zip(got, want))
