@@ -1595,7 +1595,7 @@ int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, int* pack
     if ((it + 1) % poll == 0 || it + 1 == maxit) {
       CS_HIP(hipMemcpyAsync(host_flags, c.flags, sizeof(int) * kNumFlag, hipMemcpyDeviceToHost, s));
       CS_HIP(hipStreamSynchronize(s));
-      done = host_flags[kDone] != 0;
+      done = host_flags[kDone] != 0 || host_flags[kSweepErr] != 0;
     }
   }
   if (!done) {
@@ -1641,9 +1641,10 @@ __global__ void k_save_start(Sel sel) {
   c.x1[e] = c.x[e];
 }
 
+// cloths whose solve has ended: converged, or with a wait given up
 __global__ void k_gather_done(const DevCloth* tab, int n, int* out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = tab[i].flags[kDone];
+  if (i < n) out[i] = tab[i].flags[kDone] | tab[i].flags[kSweepErr];
 }
 
 static void launch_sweep_batch(const BatchView& b, hipStream_t s) {

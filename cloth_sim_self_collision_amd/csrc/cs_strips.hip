@@ -206,7 +206,8 @@ __device__ __forceinline__ bool waiting(double imp, double rhs) {
 // them one after another made a strip trail the one before it by 2.7 us, four
 // round trips, instead of about one.
 // Past the bound on the wait the wave goes on with what it has (`gave_up`,
-// wave-uniform: it waits no more) and the solve reports the error.
+// wave-uniform: it waits no more), the launches after this one do not wait at
+// all, and the solve reports the error.
 template <bool kFwd, int K>
 __device__ __forceinline__ void set_wait(Set<K> (&q)[kSets], int n, const Sweep& w, int sub,
                                          const unsigned (&src)[3], int& gave_up) {
@@ -367,7 +368,7 @@ void k_strip_sweep(Sel sel, int polls) {
   b.src = reinterpret_cast<const int4v*>(c.st_bsrc);
   b.res = res_of(c.z, (unsigned)c.np * 24u);
   f.polls = b.polls = polls;
-  int gave_up = 0;
+  int gave_up = c.flags[kSweepErr];  // by an earlier launch
   while (true) {
     int t = 0;
     if (threadIdx.x == 0)
@@ -601,7 +602,7 @@ __global__ __launch_bounds__(kFsThreads) void k_strip_factor(Sel sel, int polls_
   if (strip == (int)gridDim.x - 1 && threadIdx.x == 0) store_device(c.st_ticket + 1, 0);
   if (strip >= c.st_nf) return;
   const int first = c.st_fptr[strip], end = c.st_fptr[strip + 1];
-  int gave_up = 0;
+  int gave_up = c.flags[kSweepErr];  // a strip before this one
   FsRow r = fs_row(c, first * kStripRows + grp), rn = fs_row(c, (first + 1) * kStripRows + grp);
   FsUpdates up;
   double av[kFsVals];

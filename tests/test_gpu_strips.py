@@ -145,6 +145,21 @@ def test_batch_steps_after_given_up_waits(sim_mod, monkeypatch):
     assert all(np.array_equal(g, w) for g, w in zip(*runs))
 
 
+def test_solve_ends_after_given_up_waits(sim_mod, monkeypatch):
+    """The iterations stop at the first convergence poll (every eight) after a
+    wait was given up, not at the cap."""
+    from cloth_sim_self_collision_amd import _lib
+    cl = _grid(33, 40)
+    monkeypatch.setenv("CLOTHSIM_STRIP_POLLS", "0")
+    with sim_mod.DeviceCloth(cl) as d, sim_mod.DeviceBatch([d]) as b:
+        for who in (d, b):
+            who.profile(True)
+            with pytest.raises(_lib.ClothSimError, match="gave up waiting"):
+                who.step(1)
+            assert who.profile_read()["ilu_sweep"][1] == 9
+            who.profile(False)
+
+
 def test_one_cloth_steps_after_given_up_waits(sim_mod, monkeypatch):
     from cloth_sim_self_collision_amd import _lib
     cl = _grid(33, 40)
