@@ -631,11 +631,12 @@ __global__ __launch_bounds__(kFsThreads) void k_strip_factor(Sel sel, int polls_
       gave_up = __builtin_amdgcn_readfirstlane(++polls >= polls_max);
     }
     wave_lds_sync();
+    bool late = false;  // this lane gave up on an update beyond the registers
     for (int k = 0; k < r.low; k++) {
 #pragma unroll
       for (int m = 0; m < kFsLayers; m++)
         if (up.code[m] >= 0 && (up.code[m] & 0xff) == k) fs_apply(sl, r.deg, up.code[m], u[m]);
-      // updates beyond the registers
+      // updates beyond the registers (a closed strip of four columns has 35 per row)
       for (int e = t + kFsLayers * kFsLanes; e < r.nu; e += kFsLanes) {
         const int cd = gptr(c.fu_code)[r.u0 + e];
         if ((cd & 0xff) != k) continue;
@@ -644,12 +645,13 @@ __global__ __launch_bounds__(kFsThreads) void k_strip_factor(Sel sel, int polls_
         do {
           asm volatile("" ::: "memory");
           fs_block(f, 72u * (unsigned)gptr(c.fu_kj)[r.u0 + e], x);
-        } while (fs_missing(x) && ++n < polls_max);
-        if (n >= polls_max) store_device(c.flags + kSweepErr, 1);
+        } while (!gave_up && !late && fs_missing(x) && ++n < polls_max);
+        late = late || n >= polls_max;
         fs_apply(sl, r.deg, cd, x);
       }
       wave_lds_sync();
     }
+    if (__builtin_amdgcn_ballot_w64(late) != 0ull) gave_up = 1;
     double* d = sl + r.deg * 9;
     if (t == 0 && r.i >= 0) {
       const double det = +d[0] * d[4] * d[8] + d[3] * d[7] * d[2] + d[6] * d[1] * d[5] -

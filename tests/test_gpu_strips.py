@@ -39,11 +39,34 @@ def _shuffled(n):
     return cl
 
 
+def _tube(m, n, copies=1, closed=False):
+    """Tubes of m vertices around and n along (closed: tori), side by side.
+    Four around: rows with 35 factor updates; 3 x 3 tori, where every vertex
+    couples to all others: 36.  A lane of the factorisation keeps updates 1 to
+    32 of a row in registers."""
+    cl = _grid(m, n * copies)
+    a, c = np.meshgrid(np.arange(m), np.arange(n if closed else n - 1))
+    p, q = c * m + a, c * m + (a + 1) % m
+    r, s = (c + 1) % n * m + a, (c + 1) % n * m + (a + 1) % m
+    tri = np.stack([p, q, s, p, s, r], -1).reshape(-1)
+    cl.tri = np.concatenate([tri + k * m * n for k in range(copies)]).astype(np.int32)
+    v = np.arange(m * n * copies)
+    t, u, k = 2 * np.pi * (v % m) / m, v // m % n, v // (m * n)
+    u = 2 * np.pi * u / n if closed else 0.02 * u
+    xyz = [0.05 * np.cos(t) + (0.1 * np.cos(u) if closed else u) + 0.4 * k,
+           0.05 * np.sin(t) + 0.3, 0.1 * np.sin(u) if closed else 0.05 * np.cos(t)]
+    cl.xyz = np.stack(xyz, -1).reshape(-1)
+    cl.xyz0 = cl.xyz.copy()
+    cl.quad = scene.bending_quads(cl.tri)
+    return cl
+
+
 MESHES = {
     "2x3": lambda: _grid(2, 3), "8x8": lambda: _grid(8, 8), "9x9": lambda: _grid(9, 9),
     "16x40": lambda: _grid(16, 40), "17x33": lambda: _grid(17, 33), "33x17": lambda: _grid(33, 17),
     "3x90": lambda: _grid(3, 90), "90x3": lambda: _grid(90, 3), "65x64": lambda: _grid(65, 64),
     "stack3x18": lambda: scene.stacked_sheets(3, 18), "shuffled20": lambda: _shuffled(20),
+    "tube4x60": lambda: _tube(4, 60), "tori3x3": lambda: _tube(3, 3, 60, True),
 }
 
 
