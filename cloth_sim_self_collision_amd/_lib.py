@@ -102,6 +102,7 @@ SIGNATURES = {
     "cs_pcg_solve": (C.c_int, [_V, _D, C.c_double, C.c_int, _D, _D, _D, _I]),
     "cs_get_bvh": (C.c_int, [_V, _I]),
     "cs_sweep_shape": (C.c_int, [_V, _I]),
+    "cs_strip_shape": (C.c_int, [_V, _I]),
     "cs_bvh_refit_prx": (C.c_int, [_V, _D, C.c_double, _D]),
     "cs_bvh_refit_ccd": (C.c_int, [_V, _D, _D, C.c_double, _D]),
     "cs_query_proximity": (C.c_int, [_V, _D, C.c_double, _I, C.c_int, _I]),

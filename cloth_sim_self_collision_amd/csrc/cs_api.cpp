@@ -1092,6 +1092,17 @@ int cs_sweep_shape(const cs_cloth* p, int* out) {
   return kOk;
 }
 
+int cs_strip_shape(const cs_cloth* p, int* out) {
+  if (!p || !out) return kBadArg;
+  const DevCloth& d = H(p)->d;
+  out[0] = strips_ok(d) ? 1 : 0;
+  out[1] = d.st_nf;
+  out[2] = d.st_nb;
+  out[3] = d.st_nf > 0 ? d.kpack : 0;
+  out[4] = d.st_ring;
+  return kOk;
+}
+
 int cs_get_bvh(const cs_cloth* p, int* nodes) {
   if (!p || !nodes) return kBadArg;
   const Cloth* c = H(p);

@@ -200,6 +200,14 @@ class DeviceCloth:
         return dict(zip(("fwd_sublevels", "bwd_sublevels", "waves", "loads_fwd", "loads_bwd",
                          "components", "quad", "wave_loads"), out))
 
+    def strip_shape(self) -> dict:
+        """The strip plan of the ILU sweeps (cs_strip_shape): whether the
+        launched sweeps go by strips, strips forward and backward, blocks per
+        row, sub-levels in the LDS ring."""
+        out = (C.c_int * 5)()
+        check(_lib.load().cs_strip_shape(self.h, out))
+        return dict(zip(("strips", "forward", "backward", "blocks", "ring"), out))
+
     def profile_read(self) -> dict:
         out = {}
         for k, name in enumerate(self.PROFILE_KINDS):

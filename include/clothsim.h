@@ -347,6 +347,11 @@ int cs_issue_probe(int waves, int steps, double* ns_per_load);
  * its busiest workgroup (forward and backward; waves without a row in three
  * consecutive sub-levels skip their loads) */
 int cs_sweep_shape(const cs_cloth* cloth, int* out);
+/* the strip plan of a cloth's ILU sweeps: out[5] = 1 if the mesh and the
+ * options have the launched sweeps go by strips, strips of the forward and of
+ * the backward sweep, blocks per row, sub-levels in the LDS ring (0 without a
+ * plan) */
+int cs_strip_shape(const cs_cloth* cloth, int* out);
 
 #ifdef __cplusplus
 }

@@ -1,5 +1,5 @@
 // Host-only check of the per-mesh setup and its cache (run under ASan/UBSan):
-//   setup_check <mesh.bin> <cache dir>
+//   setup_check <mesh.bin> <cache dir> [blocks ring strips]
 // mesh.bin: int32 np, nt, nq; double xyz[3np]; int32 tri[3nt], quad[4nq].
 // 1. build_setup, then validate_setup must accept it;
 // 2. planted mistakes in copies of the setup (an index out of range, a ring
@@ -7,12 +7,14 @@
 //    child out of range, a gather source past the elements) must each be
 //    rejected;
 // 3. the strip plan of the sweeps, when the mesh has one, passes its own
-//    validator, and a planted ring offset does not;
+//    validator, and a planted ring offset does not; with the last three
+//    arguments it is the plan they name (zeros: the mesh has none);
 // 4. through the cache: a miss writes the file, a second lookup hits and
 //    returns the same setup, a file with one flipped payload byte is
 //    rejected and rebuilt (a miss), and the rebuilt setup equals the fresh one.
 // Prints "ok" and exits 0 when every check holds.
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -38,7 +40,8 @@ static bool same(const MeshSetup& a, const MeshSetup& b) {
 }
 
 int main(int argc, char** argv) {
-  if (argc != 3) return fail("usage: setup_check mesh.bin cachedir");
+  if (argc != 3 && argc != 6)
+    return fail("usage: setup_check mesh.bin cachedir [blocks ring strips]");
   FILE* f = std::fopen(argv[1], "rb");
   if (!f) return fail("cannot open mesh");
   int hdr[3];
@@ -92,6 +95,14 @@ int main(int argc, char** argv) {
   // written to; a planted offset or import is caught
   cs::StripPlan strips;
   cs::build_strips(s, strips);
+  if (argc == 6) {
+    const int got[3] = {strips.ok ? strips.k : 0, strips.ok ? strips.ring : 0,
+                        strips.ok ? (int)strips.fwd.ptr.size() - 1 : 0};
+    for (int k = 0; k < 3; k++)
+      if (got[k] != std::atoi(argv[3 + k]))
+        return fail("another strip plan than expected: " + std::to_string(got[0]) + " blocks, ring " +
+                    std::to_string(got[1]) + ", " + std::to_string(got[2]) + " strips");
+  }
   if (strips.ok) {
     err = cs::validate_strips(s, strips);
     if (!err.empty()) return fail(err);

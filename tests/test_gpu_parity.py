@@ -360,9 +360,9 @@ def test_velocity_update_and_host_obstacle_values(sim_mod, oracle_mod):
         assert (pd + cl.clearance > 0).any()  # the obstacle term is active
 
 
-# (scene, steps, sweep variant, PCG variant): sweep 0 = packed quad sweep,
-# 1 = row-by-row; PCG 0 = automatic (one launch per PCG operation), 2 = the
-# whole solve in one workgroup
+# (scene, steps, sweep variant, PCG variant): sweep 0 = automatic (these meshes:
+# by strips), 1 = row-by-row; PCG 0 = automatic (one launch per PCG operation),
+# 2 = the whole solve in one workgroup (packed one-workgroup sweeps)
 @pytest.mark.parametrize("name,steps,variant,pcg", [
     ("drape32", 100, 0, 0), ("drape32", 100, 0, 2), ("refdemo0", 60, 0, 0),
     ("refdemo1", 60, 0, 2), ("fold24", 60, 0, 0), ("fold24", 60, 0, 2),

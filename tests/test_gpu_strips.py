@@ -1,15 +1,16 @@
-"""The triangular sweeps by strips against the oracle and the row-by-row sweep.
-
-One M^-1 r with a random right-hand side on grids whose sides sit at the edges
-of a strip (eight rows per sub-level): one strip, one row more, ragged last
-strips, long and short columns, several components, and a mesh with shuffled
-vertex numbers (its strips import most of their rows, or the mesh does not fit
-strips at all).  Each operation is one IEEE rounding in the reference's order,
-so the comparison is exact."""
+"""The triangular sweeps and the factorisation by strips against the oracle,
+on meshes whose plans cover each kernel instance: grids whose sides sit at the
+edges of a strip (eight rows per sub-level; one strip, one row more, ragged
+last strips, several components), renumbered grids (seven and eight blocks per
+row, rings of 16 and 32 sub-levels, imports many sub-levels ahead), rows with
+more than 32 factor updates, and meshes without a strip plan, which take the
+packed one-workgroup sweep or the row-by-row sweep.  Which path a mesh takes is
+part of each test.  Each operation is one IEEE rounding in the reference's
+order, so the comparisons are exact."""
 import numpy as np
 import pytest
 
-from cloth_sim_self_collision_amd import scene
+from _meshes import MESHES, QUAD, ROWS, grid as _grid
 
 pytestmark = pytest.mark.gpu
 
@@ -22,60 +23,25 @@ def sim_mod():
     return sim
 
 
-def _grid(nx, ny):
-    return scene.drop_on_obstacle(nx, 0.4, scene.sphere((0.0, 0.0, 0.0), 0.3), ny=ny, seed=nx + ny)
-
-
-def _shuffled(n):
-    """A square grid with its vertices renumbered at random."""
-    cl = _grid(n, n)
-    perm = np.random.default_rng(n).permutation(cl.np_).astype(np.int32)
-    inv = np.empty_like(perm)
-    inv[perm] = np.arange(cl.np_, dtype=np.int32)
-    cl.xyz0 = cl.xyz0.reshape(-1, 3)[perm].reshape(-1).copy()
-    cl.xyz = cl.xyz.reshape(-1, 3)[perm].reshape(-1).copy()
-    cl.tri = inv[cl.tri]
-    cl.quad = scene.bending_quads(cl.tri)
-    return cl
-
-
-def _tube(m, n, copies=1, closed=False):
-    """Tubes of m vertices around and n along (closed: tori), side by side.
-    Four around: rows with 35 factor updates; 3 x 3 tori, where every vertex
-    couples to all others: 36.  A lane of the factorisation keeps updates 1 to
-    32 of a row in registers."""
-    cl = _grid(m, n * copies)
-    a, c = np.meshgrid(np.arange(m), np.arange(n if closed else n - 1))
-    p, q = c * m + a, c * m + (a + 1) % m
-    r, s = (c + 1) % n * m + a, (c + 1) % n * m + (a + 1) % m
-    tri = np.stack([p, q, s, p, s, r], -1).reshape(-1)
-    cl.tri = np.concatenate([tri + k * m * n for k in range(copies)]).astype(np.int32)
-    v = np.arange(m * n * copies)
-    t, u, k = 2 * np.pi * (v % m) / m, v // m % n, v // (m * n)
-    u = 2 * np.pi * u / n if closed else 0.02 * u
-    xyz = [0.05 * np.cos(t) + (0.1 * np.cos(u) if closed else u) + 0.4 * k,
-           0.05 * np.sin(t) + 0.3, 0.1 * np.sin(u) if closed else 0.05 * np.cos(t)]
-    cl.xyz = np.stack(xyz, -1).reshape(-1)
-    cl.xyz0 = cl.xyz.copy()
-    cl.quad = scene.bending_quads(cl.tri)
-    return cl
-
-
-MESHES = {
-    "2x3": lambda: _grid(2, 3), "8x8": lambda: _grid(8, 8), "9x9": lambda: _grid(9, 9),
-    "16x40": lambda: _grid(16, 40), "17x33": lambda: _grid(17, 33), "33x17": lambda: _grid(33, 17),
-    "3x90": lambda: _grid(3, 90), "90x3": lambda: _grid(90, 3), "65x64": lambda: _grid(65, 64),
-    "stack3x18": lambda: scene.stacked_sheets(3, 18), "shuffled20": lambda: _shuffled(20),
-    "tube4x60": lambda: _tube(4, 60), "tori3x3": lambda: _tube(3, 3, 60, True),
-}
+def _mesh(name, d=None):
+    """The mesh, or with its device cloth: the sweeps take the expected path."""
+    make, want = MESHES[name]
+    if d is None:
+        return make()
+    got = d.strip_shape()
+    if want in (QUAD, ROWS):
+        assert not got["strips"] and d.sweep_shape()["quad"] == (want == QUAD)
+    else:
+        assert got["strips"] and (got["blocks"], got["ring"], got["forward"]) == want
 
 
 @pytest.mark.parametrize("name", sorted(MESHES))
 def test_solve_by_strips_bitwise(sim_mod, oracle_mod, name):
-    cl = MESHES[name]()
+    cl = _mesh(name)
     o = oracle_mod.Oracle(cl, "port")
     rng = np.random.default_rng(len(name))
     with sim_mod.DeviceCloth(cl) as d:
+        _mesh(name, d)
         dia, crs, b = d.assemble(cl.xyz, cl.uvw)
         d.ilu_factor()
         fd, fc = d.get_factor()
@@ -84,6 +50,7 @@ def test_solve_by_strips_bitwise(sim_mod, oracle_mod, name):
             d.set_option(1, 0)
             strips = d.ilu_solve(v)
             d.set_option(1, 1)
+            assert not d.strip_shape()["strips"]
             rows = d.ilu_solve(v)
             assert np.array_equal(strips, rows)
             assert np.array_equal(strips, o.ilu_solve(fd, fc, v))
@@ -96,9 +63,79 @@ def test_solve_by_strips_bitwise(sim_mod, oracle_mod, name):
         assert np.array_equal(strips, d.ilu_solve(v), equal_nan=True)
 
 
-def test_solves_of_each_layout_alternate(sim_mod):
+def _fp32(fc):
+    return fc.astype(np.float32).astype(np.float64)
+
+
+@pytest.mark.parametrize("name", sorted(n for n in MESHES if MESHES[n][1] != ROWS))
+def test_mixed_precision_solve_bitwise(sim_mod, oracle_mod, name):
+    """Mixed precision rounds the sweeps' coefficients to FP32 and nothing
+    else: the oracle's solve with the rounded blocks, exactly."""
+    cl = _mesh(name)
+    o = oracle_mod.Oracle(cl, "port")
+    rng = np.random.default_rng(len(name))
+    with sim_mod.DeviceCloth(cl) as d:
+        d.assemble(cl.xyz, cl.uvw)
+        d.ilu_factor()
+        fd, fc = d.get_factor()
+        d.set_option(3, 1)
+        _mesh(name, d)
+        for k in range(2):
+            v = rng.standard_normal(3 * cl.np_)
+            assert np.array_equal(d.ilu_solve(v), o.ilu_solve(fd, _fp32(fc), v))
+
+
+BATCHES = {  # members share the blocks per row; one without a plan: none by strips
+    "K7": ["morton64", "jitter24a", "tube4x60"],
+    "K8": ["jitter24c", "jitter40", "jitter24b"],
+    "K7quad": ["jitter40far", "morton64", "jitter24a"],
+    "K6": ["65x64", "8x8", "stack3x18"],
+    "rows": ["8x8", "shuffled20"],
+}
+
+
+@pytest.mark.parametrize("batch", sorted(BATCHES))
+@pytest.mark.parametrize("prec", [0, 1])
+def test_steps_alone_and_in_a_batch_bitwise(sim_mod, oracle_mod, batch, prec):
+    """Two internal steps of plans with different rings side by side: each
+    cloth ends as it does alone, in FP64 as the oracle's."""
+    names = BATCHES[batch]
+    if prec and any(MESHES[n][1] == ROWS for n in names):
+        pytest.skip("the row-by-row sweep is FP64 only")
+    cls = [_mesh(n) for n in names]
+    for c in cls:
+        c.pcg_maxit = 30
+    alone = []
+    for n, cl in zip(names, cls):
+        with sim_mod.DeviceCloth(cl) as d:
+            d.set_option(3, prec)
+            _mesh(n, d)
+            d.step(2)
+            alone.append(d.get_state())
+        if not prec:
+            o = oracle_mod.Oracle(cl, "port")
+            x, v = cl.xyz.copy(), cl.uvw.copy()
+            for _ in range(2):
+                x, v, *_ = o.step(x, v)
+            assert np.array_equal(alone[-1][0], x) and np.array_equal(alone[-1][1], v), n
+    devs = [sim_mod.DeviceCloth(c) for c in cls]
+    try:
+        for d in devs:
+            d.set_option(3, prec)
+        with sim_mod.DeviceBatch(devs) as b:
+            b.step(2)
+        for n, d, (x, v) in zip(names, devs, alone):
+            gx, gv = d.get_state()
+            assert np.array_equal(gx, x) and np.array_equal(gv, v), n
+    finally:
+        for d in devs:
+            d.close()
+
+
+@pytest.mark.parametrize("name", ["17x33", "jitter24a", "jitter24c", "jitter40far"])
+def test_solves_of_each_layout_alternate(sim_mod, name):
     """The packed copies of one factor follow the solve that needs them."""
-    cl = _grid(20, 24)
+    cl = _mesh(name)
     with sim_mod.DeviceCloth(cl) as d:
         _, _, b = d.assemble(cl.xyz, cl.uvw)
         d.ilu_factor()
@@ -121,10 +158,11 @@ def test_solves_of_each_layout_alternate(sim_mod):
 def test_factor_by_strips_bitwise(sim_mod, oracle_mod, name):
     """The factorisation on the same meshes, on the assembled system and on a
     random one (other update patterns of magnitude), twice each."""
-    cl = MESHES[name]()
+    cl = _mesh(name)
     o = oracle_mod.Oracle(cl, "port")
     rng = np.random.default_rng(3)
     with sim_mod.DeviceCloth(cl) as d:
+        _mesh(name, d)
         dia, crs, b = d.assemble(cl.xyz, cl.uvw)
         rdia = rng.standard_normal(dia.shape) + np.tile(9.0 * np.eye(3).reshape(-1), cl.np_)
         rcrs = rng.standard_normal(crs.shape)

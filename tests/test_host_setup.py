@@ -12,6 +12,7 @@ import subprocess
 import numpy as np
 import pytest
 
+from _meshes import MESHES, QUAD, ROWS
 from cloth_sim_self_collision_amd import scene
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -73,4 +74,21 @@ def test_setup_validates_and_cache_rejects_corruption(checker, tmp_path, name):
                UBSAN_OPTIONS="print_stacktrace=1")
     r = subprocess.run([checker, str(mesh), str(cache)], capture_output=True, text=True,
                        timeout=300, env=env)
+    assert r.returncode == 0 and r.stdout.startswith("ok"), r.stdout + r.stderr
+
+
+@pytest.mark.parametrize("name", sorted(MESHES))
+def test_meshes_have_the_expected_strip_plan(checker, tmp_path, name):
+    """A mesh that stops fitting the strips, or fits them otherwise, is seen
+    here: its sweeps would take another path with the same results."""
+    make, want = MESHES[name]
+    if want in (QUAD, ROWS):
+        want = (0, 0, 0)
+    mesh = tmp_path / "mesh.bin"
+    _write_mesh(mesh, make())
+    cache = tmp_path / "cache"
+    cache.mkdir()
+    r = subprocess.run([checker, str(mesh), str(cache)] + [str(v) for v in want],
+                       capture_output=True, text=True, timeout=300,
+                       env=dict(os.environ, ASAN_OPTIONS="detect_leaks=1:abort_on_error=0"))
     assert r.returncode == 0 and r.stdout.startswith("ok"), r.stdout + r.stderr
