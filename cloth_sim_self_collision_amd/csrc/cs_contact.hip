@@ -541,25 +541,20 @@ __device__ __forceinline__ void vel_add(double* U, int i, double a, double b, do
   U[3 * i + 2] += d;
 }
 
-__device__ void impulse_one(const int* e, const double* X, double* U, double delta, double k,
-                            double dt, double m, int ccd) {
+// the impulse of a continuous contact
+__device__ void impulse_ccd(const int* e, const double* X, double* U, double delta, double dt,
+                            double m) {
   const int i0 = e[1], i1 = e[2], i2 = e[3], i3 = e[4];
   const Vec3 p0 = at(X, i0), p1 = at(X, i1), p2 = at(X, i2), p3 = at(X, i3);
   const Vec3 v0 = at(U, i0), v1 = at(U, i1), v2 = at(U, i2), v3 = at(U, i3);
-  double t = 0;
-  if (ccd) {
-    // end positions are p + v, not p + dt v (self_collision_cloth.cpp:141)
-    t = coplanar_time(p0, p1, p2, p3, p0 + v0, p1 + v1, p2 + v2, p3 + v3);
-    if (t < 0 || t > 1) return;
-  }
+  // end positions are p + v, not p + dt v (self_collision_cloth.cpp:141)
+  const double t = coplanar_time(p0, p1, p2, p3, p0 + v0, p1 + v1, p2 + v2, p3 + v3);
+  if (t < 0 || t > 1) return;
   if (e[0]) {  // face (i0,i1,i2) - vertex i3
     double w0, w1;
     {
-      double dist;
-      if (ccd)
-        dist = face_vertex(p0 + t * v0, p1 + t * v1, p2 + t * v2, p3 + t * v3, w0, w1);
-      else
-        dist = face_vertex(p0, p1, p2, p3, w0, w1);
+      const double dist =
+          face_vertex(p0 + t * v0, p1 + t * v1, p2 + t * v2, p3 + t * v3, w0, w1);
       if (w0 < 0 || w0 > 1) return;
       if (w1 < 0 || w1 > 1) return;
       if (dist > delta) return;
@@ -568,23 +563,11 @@ __device__ void impulse_one(const int* e, const double* X, double* U, double del
     const Vec3 pc = w0 * p0 + w1 * p1 + w2 * p2;
     const Vec3 nrm = unit(p3 - pc);
     const double rel = dot(v3 - w0 * v0 - w1 * v1 - w2 * v2, nrm);
-    double j;
-    if (!ccd) {
-      const double depth = delta - dot(p3 - pc, nrm);
-      if (rel > 0.1 * depth / dt) return;
-      const double el = dt * k * depth;
-      const double ie = m * (0.1 * depth / dt - rel);
-      const double imin = (el < ie) ? el : ie;
-      j = 2 * imin / (1 + w0 * w0 + w1 * w1 + w2 * w2);
-      j /= m;
-      j *= 0.25;
-    } else {
-      if (rel > 0.1 * delta / dt) return;
-      const double imp = m * (0.1 * delta / dt - rel);
-      j = 2 * imp / (1.0 + w0 * w0 + w1 * w1 + w2 * w2);
-      j /= m;
-      j *= 0.1;
-    }
+    if (rel > 0.1 * delta / dt) return;
+    const double imp = m * (0.1 * delta / dt - rel);
+    double j = 2 * imp / (1.0 + w0 * w0 + w1 * w1 + w2 * w2);
+    j /= m;
+    j *= 0.1;
     vel_add(U, i0, -nrm.x * j * w0, -nrm.y * j * w0, -nrm.z * j * w0);
     vel_add(U, i1, -nrm.x * j * w1, -nrm.y * j * w1, -nrm.z * j * w1);
     vel_add(U, i2, -nrm.x * j * w2, -nrm.y * j * w2, -nrm.z * j * w2);
@@ -592,11 +575,7 @@ __device__ void impulse_one(const int* e, const double* X, double* U, double del
   } else {  // edge (i0,i1) - edge (i2,i3)
     double wa, wb;
     {
-      double dist;
-      if (ccd)
-        dist = edge_edge(p0 + t * v0, p1 + t * v1, p2 + t * v2, p3 + t * v3, wa, wb);
-      else
-        dist = edge_edge(p0, p1, p2, p3, wa, wb);
+      const double dist = edge_edge(p0 + t * v0, p1 + t * v1, p2 + t * v2, p3 + t * v3, wa, wb);
       if (wa < 0 || wa > 1) return;
       if (wb < 0 || wb > 1) return;
       if (dist > delta) return;
@@ -605,23 +584,11 @@ __device__ void impulse_one(const int* e, const double* X, double* U, double del
     const Vec3 cb = (1 - wb) * p2 + wb * p3;
     const Vec3 nrm = unit(cb - ca);
     const double rel = dot((1 - wb) * v2 + wb * v3 - (1 - wa) * v0 - wa * v1, nrm);
-    double j;
-    if (!ccd) {
-      const double depth = delta - norm(cb - ca);
-      if (rel > 0.1 * depth / dt) return;
-      const double el = dt * k * depth;
-      const double ie = m * (0.1 * depth / dt - rel);
-      const double imin = (el < ie) ? el : ie;
-      j = 2 * imin / (wa * wa + (1 - wa) * (1 - wa) + wb * wb + (1 - wb) * (1 - wb));
-      j /= m;
-      j *= 0.25;
-    } else {
-      if (rel > 0.1 * delta / dt) return;
-      const double imp = m * (0.1 * delta / dt - rel);
-      j = 2 * imp / (wa * wa + (1 - wa) * (1 - wa) + wb * wb + (1 - wb) * (1 - wb));
-      j /= m;
-      j *= 0.1;
-    }
+    if (rel > 0.1 * delta / dt) return;
+    const double imp = m * (0.1 * delta / dt - rel);
+    double j = 2 * imp / (wa * wa + (1 - wa) * (1 - wa) + wb * wb + (1 - wb) * (1 - wb));
+    j /= m;
+    j *= 0.1;
     vel_add(U, i0, -nrm.x * j * (1 - wa), -nrm.y * j * (1 - wa), -nrm.z * j * (1 - wa));
     vel_add(U, i1, -nrm.x * j * wa, -nrm.y * j * wa, -nrm.z * j * wa);
     vel_add(U, i2, +nrm.x * j * (1 - wb), +nrm.y * j * (1 - wb), +nrm.z * j * (1 - wb));
@@ -631,8 +598,8 @@ __device__ void impulse_one(const int* e, const double* X, double* U, double del
 
 // What a proximity impulse takes from the positions alone: formed for every
 // contact at once before the sequential schedule, whose chain then holds only
-// the velocities (impulse_one does both for the continuous passes, where the
-// time of impact depends on the velocities).  One 128-byte line per contact.
+// the velocities (in the continuous passes the time of impact depends on them:
+// impulse_ccd).  One 128-byte line per contact.
 struct alignas(128) ImpulseGeom {
   double c[4];     // weights of the four velocities (face-vertex: c[3] is 1)
   double n[3];     // contact normal
@@ -689,8 +656,8 @@ __global__ void k_impulse_geom(const int* ce, int g, const double* X, double del
   out[i] = o;
 }
 
-// the velocity part of a proximity impulse: impulse_one's operations in its
-// order (its ccd == 0 branches)
+// the velocity part of a proximity impulse, the reference's operations in its
+// order
 __device__ __forceinline__ void impulse_velocity(const ImpulseGeom& o, Vec3 v0, Vec3 v1, Vec3 v2,
                                                  Vec3 v3, double* U, double m) {
   if (o.kind == 0) return;
@@ -786,29 +753,41 @@ __device__ __forceinline__ void lds_only_barrier() {
 // round, after the barrier that ends this one) and loads its velocities;
 // behind an LDS-only barrier the runners form and store the impulses while the
 // fetchers load the released contacts' geometry and successors, which come
-// from far memory, into LDS for the next round.  The four counter atomics of a
-// contact are all in flight together, at workgroup scope (no other workgroup
-// touches the counters).  Per round 2.2 us, from 3.6 with every contact
-// loading its own data: folded 256^2 sheet 6.8 ms from 11.4, 253 x 397 drop
-// 20 from 27, four stacked 128^2 sheets 6.4 from 7.4.
+// from far memory, into LDS for the next round, every load of a thread in
+// flight at once.  The four counter atomics of a contact are all in flight
+// together, at workgroup scope (no other workgroup touches the counters).
+// What a round has beyond the runners' contacts every thread helps to run
+// first.  In a continuous pass, where nothing can be fetched ahead (the
+// geometry depends on the velocities), every thread runs contacts.
+// Against 1024 threads that each load their own data, and against 256 runners
+// with one load of a fetcher in flight: folded 256^2 sheet 14.8 / 7.1 / 6.6 ms
+// (2.1 us per round), 253 x 397 drop 38 / 20.1 / 18.2 ms, four stacked 128^2
+// sheets 10.1 / 6.4 / 5.1 ms, and four stacked 512^2 sheets, whose 23 035
+// rounds have about 290 contacts, 215 / 259 / 193 ms; 384 runners: 7.4, 20.1,
+// 5.5 and 204 ms.
 // Released contacts are listed in LDS up to lds_cap, the rest of a longer round
-// in the global lists; the first kDrainRecs of a round have their data in LDS,
-// others load it themselves.  lds_cap (at most kDrainLds) is smaller only for
+// in the global lists; the first kDrainRecs of a round have their data in LDS
+// (two rounds of them and the lists fill 140 of 160 KB), others load it
+// themselves.  lds_cap (at most kDrainLds) is smaller only for
 // tests (the CLOTHSIM_DRAIN_LDS environment variable).
 constexpr int kDrainLds = 4096;
-constexpr int kDrainRun = 256;    // threads that run contacts, and as many that fetch
-constexpr int kDrainRecs = 256;   // contacts of a round whose data is in LDS
+constexpr int kDrainRun = 512;   // runners, and as many fetchers
+constexpr int kDrainRecs = 384;  // contacts of a round whose data is in LDS
 constexpr int kDrainPieces = (int)sizeof(ImpulseGeom) / 16 + 1;  // 16 bytes each: geometry, successors
+constexpr int kDrainCcd = 1024;  // threads of a continuous pass
+static_assert(sizeof(ImpulseGeom) % 16 == 0, "a contact's geometry moves in 16-byte pieces");
 
-__global__ __launch_bounds__(2 * kDrainRun) void k_impulse_drain(
+// kGeom: a proximity pass (else a continuous one, which reads ce, X, delta, dt)
+template <bool kGeom>
+__global__ __launch_bounds__(kGeom ? 2 * kDrainRun : kDrainCcd) void k_impulse_drain(
     const int* ce, const int* succ, int* npred, int* ready0, int* ready1, const double* X, double* U,
-    double delta, double k, double dt, double m, int ccd, int* counters, int lds_cap,
-    const ImpulseGeom* geom) {
+    double delta, double dt, double m, int* counters, int lds_cap, const ImpulseGeom* geom) {
+  constexpr int kThreads = kGeom ? 2 * kDrainRun : kDrainCcd;
+  constexpr int kRun = kGeom ? kDrainRun : 0;  // contacts of a round that the runners take
   __shared__ int count[2];  // contacts released for the next round, in turn
   __shared__ int lists[2][kDrainLds];
-  __shared__ int4 rec[2][kDrainRecs][kDrainPieces];
+  __shared__ int4 rec[2][kGeom ? kDrainRecs : 1][kDrainPieces];
   const int tid = threadIdx.x;
-  const bool runner = tid < kDrainRun;
   int n = counters[kReady];
   int *gcur = ready0, *gnxt = ready1;  // the first round's list and the spills
   int cur = 0;                         // the LDS list and data of this round
@@ -819,6 +798,7 @@ __global__ __launch_bounds__(2 * kDrainRun) void k_impulse_drain(
   const int recs = min(kDrainRecs, lds_cap);
   if (tid < 2) count[tid] = 0;
   __syncthreads();
+  auto listed = [&](int t) { return (first || t >= lds_cap) ? gcur[t] : lists[cur][t]; };
   auto release = [&](int c) {
     const int pos = atomicAdd(&count[cur ^ 1], 1);
     if (pos < lds_cap)
@@ -836,60 +816,65 @@ __global__ __launch_bounds__(2 * kDrainRun) void k_impulse_drain(
       // successor the contact's own counter, which nothing reads any more
       left[a] = __hip_atomic_fetch_sub(&npred[s4[a] >= 0 ? s4[a] : i], 1, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_WORKGROUP);
-    if (geom)
+    if (kGeom)
+#pragma unroll
       for (int a = 0; a < 4; a++) v[a] = at(U, o.v[a]);
 #pragma unroll
     for (int a = 0; a < 4; a++)
       if (s4[a] >= 0 && left[a] == 1) release(s4[a]);
   };
   auto finish = [&](int i, const ImpulseGeom& o, const Vec3 (&v)[4]) {
-    if (geom)
+    if (kGeom)
       impulse_velocity(o, v[0], v[1], v[2], v[3], U, m);
     else
-      impulse_one(ce + 5 * i, X, U, delta, k, dt, m, ccd);
+      impulse_ccd(ce + 5 * i, X, U, delta, dt, m);
   };
   while (n > 0) {
     ImpulseGeom o{};
     Vec3 v[4];
     int i = -1;
-    if (runner) {
-      // all but the last of this thread's contacts of a wide round
-      int t = tid;
-      for (; t + kDrainRun < n; t += kDrainRun) {
-        const int c = (first || t >= lds_cap) ? gcur[t] : lists[cur][t];
-        if (geom) o = geom[c];
-        begin(c, reinterpret_cast<const int4*>(succ)[c], o, v);
-        finish(c, o, v);
-      }
-      if (t < n) {
-        i = (first || t >= lds_cap) ? gcur[t] : lists[cur][t];
-        int4 sc;
-        if (geom && !first && t < recs) {
-          int4 w[kDrainPieces];
+    // what the runners do not take, on every thread
+    for (int t = kRun + tid; t < n; t += kThreads) {
+      const int c = listed(t);
+      if (kGeom) o = geom[c];
+      begin(c, reinterpret_cast<const int4*>(succ)[c], o, v);
+      finish(c, o, v);
+    }
+    if (kGeom && tid < min(n, kRun)) {
+      i = listed(tid);
+      int4 sc;
+      if (!first && tid < recs) {
+        int4 w[kDrainPieces];
 #pragma unroll
-          for (int p = 0; p < kDrainPieces; p++) w[p] = rec[cur][t][p];
-          __builtin_memcpy(&o, w, sizeof(o));
-          sc = w[kDrainPieces - 1];
-        } else {
-          if (geom) o = geom[i];
-          sc = reinterpret_cast<const int4*>(succ)[i];
-        }
-        begin(i, sc, o, v);
+        for (int p = 0; p < kDrainPieces; p++) w[p] = rec[cur][tid][p];
+        __builtin_memcpy(&o, w, sizeof(o));
+        sc = w[kDrainPieces - 1];
+      } else {
+        o = geom[i];
+        sc = reinterpret_cast<const int4*>(succ)[i];
       }
+      begin(i, sc, o, v);
     }
     lds_only_barrier();  // the next round's list is complete; loads stay in flight
     const int next = count[cur ^ 1];
-    if (runner) {
-      if (i >= 0) finish(i, o, v);
-      if (tid == 0) count[cur] = 0;  // read by every thread before the barrier above
-    } else if (geom) {
-      const int pieces = min(next, recs) * kDrainPieces;
-      for (int q = tid - kDrainRun; q < pieces; q += kDrainRun) {
+    if (i >= 0) finish(i, o, v);
+    if (tid == 0) count[cur] = 0;  // read by every thread before the barrier above
+    const int pieces = min(next, recs) * kDrainPieces;
+    if (kGeom && tid - kRun >= 0 && tid - kRun < pieces) {
+      // every load issued before the first is stored (past the end: the last piece)
+      int4 w[kDrainPieces];
+#pragma unroll
+      for (int u = 0; u < kDrainPieces; u++) {
+        const int q = min(tid - kRun + u * kDrainRun, pieces - 1);
         const int e = q / kDrainPieces, p = q - e * kDrainPieces;
         const int c = lists[cur ^ 1][e];
-        rec[cur ^ 1][e][p] = p < kDrainPieces - 1
-                                 ? reinterpret_cast<const int4*>(geom + c)[p]
-                                 : reinterpret_cast<const int4*>(succ)[c];
+        w[u] = p < kDrainPieces - 1 ? reinterpret_cast<const int4*>(geom + c)[p]
+                                    : reinterpret_cast<const int4*>(succ)[c];
+      }
+#pragma unroll
+      for (int u = 0; u < kDrainPieces; u++) {
+        const int q = tid - kRun + u * kDrainRun;
+        if (q < pieces) (&rec[cur ^ 1][0][0])[q] = w[u];
       }
     }
     done += n;
@@ -1309,9 +1294,14 @@ int impulses(ContactState& cs, const DevCloth& d, const Params& P, hipStream_t s
   }
   int lds_cap = kDrainLds;
   if (const char* e = getenv("CLOTHSIM_DRAIN_LDS")) lds_cap = std::min(std::max(atoi(e), 1), kDrainLds);
-  hipLaunchKernelGGL(k_impulse_drain, dim3(1), dim3(2 * kDrainRun), 0, s, cs.ce, cs.succ, cs.npred,
-                     cs.ready[0], cs.ready[1], X, U, P.clearance, P.k_contact, P.dt, P.mass, ccd,
-                     cs.counters, lds_cap, ccd ? nullptr : (const ImpulseGeom*)cs.geom);
+  if (ccd)
+    hipLaunchKernelGGL(k_impulse_drain<false>, dim3(1), dim3(kDrainCcd), 0, s, cs.ce, cs.succ,
+                       cs.npred, cs.ready[0], cs.ready[1], X, U, P.clearance, P.dt, P.mass,
+                       cs.counters, lds_cap, (const ImpulseGeom*)nullptr);
+  else
+    hipLaunchKernelGGL(k_impulse_drain<true>, dim3(1), dim3(2 * kDrainRun), 0, s, cs.ce, cs.succ,
+                       cs.npred, cs.ready[0], cs.ready[1], X, U, P.clearance, P.dt, P.mass,
+                       cs.counters, lds_cap, (const ImpulseGeom*)cs.geom);
   CS_HIP(hipGetLastError());
   if (int st = read_counters(cs, s)) return st;
   if (cs.hcounters[kDoneCnt] != g) {

@@ -387,6 +387,30 @@ def test_trajectory_bitwise(sim_mod, oracle_mod, name, steps, variant, pcg):
             del x_before
 
 
+@pytest.mark.parametrize("lds", [None, 100])
+@pytest.mark.parametrize("n,clearance,gap,closing", [(96, 1.05, 0.9, 0.0), (64, 0.05, 0.5, 0.28)])
+def test_wide_impulse_rounds(sim_mod, oracle_mod, monkeypatch, n, clearance, gap, closing, lds):
+    """Two sheets with randomly numbered vertices: proximity rounds of up to
+    605 contacts (more than the 512 that have a thread of their own and the
+    384 whose data is fetched ahead) and continuous ones of up to 281, with
+    every round's list in LDS or all but 100 of it in the global lists."""
+    from _meshes import renumbered
+    h = 1.0 / (n - 1)
+    cl = scene.stacked_sheets(2, n, gap=gap * h, z0=1.0, jitter=0.05 * h, clearance=clearance * h)
+    cl = renumbered(cl, np.random.default_rng(1).permutation(cl.np_))
+    z = cl.xyz.reshape(-1, 3)[:, 2]
+    cl.uvw.reshape(-1, 3)[:, 2] = np.where(z > z.mean(), -closing, closing) * h / cl.dt
+    v, applied = oracle_mod.Oracle(cl, "port").contact_resolve(cl.xyz, cl.uvw)
+    if lds:
+        monkeypatch.setenv("CLOTHSIM_DRAIN_LDS", str(lds))
+    with sim_mod.DeviceCloth(cl) as d:
+        d.set_step_start(cl.xyz)
+        got, st = d.intermediate_velocity_contact_resolved()
+        assert got == applied
+        assert st["n_prox"] == 81999 if n == 96 else st["n_ccd"][0] == 34218
+        assert np.array_equal(d.get_state()[1], v)
+
+
 def test_impulse_rounds_through_the_global_lists(sim_mod, oracle_mod, monkeypatch):
     """The impulse worklist keeps each round's list in LDS up to a capacity
     and the rest of a wider round in global memory; with the capacity cut to
