@@ -138,6 +138,7 @@ struct Cloth {
   Params P;
   DevCloth d;
   Arena arena;
+  Arena quad;  // the packed factor of the one-workgroup sweeps, once needed (packed_arrays)
   hipStream_t stream = nullptr;
   int* hflags = nullptr;  // pinned
   double* hscal = nullptr;
@@ -194,6 +195,23 @@ int check_params(const cs_params* p) {
     set_error("unknown obstacle kind");
     return kBadArg;
   }
+  return kOk;
+}
+
+// The packed factor's arrays (about 1 KB per vertex), which the solves that do
+// not go by strips use: allocated for meshes without a strip plan, and once an
+// option or a batch asks for such a solve.
+int packed_arrays(Cloth* c) {
+  DevCloth& d = c->d;
+  if (d.f_blk) return kOk;
+  // value pairs per lane: (3 k + 1) / 2 pairs of 3 lanes x 2 doubles per slot
+  const size_t pk = (size_t)(3 * d.kpack + 1) / 2 * 6 * d.np;
+  Arena q;
+  q.reserve(&d.f_blk, pk);
+  q.reserve(&d.f_dinv, d.kpack ? 12 * (size_t)d.np : 0);
+  q.reserve(&d.b_blk, pk);
+  if (int st = q.commit(c->stream)) return st;
+  c->quad = q;
   return kOk;
 }
 
@@ -298,11 +316,6 @@ int build(Cloth* c, const cs_mesh* m) {
   A.reserve(&brc, kl ? 2 * (size_t)np : 0);
   A.reserve(&bmeta, kl ? (size_t)meta_groups(std::max(kl, ku)) * 8 * np : 0);
   const int kq = kl > 0 ? std::max(kl, ku) : 0;
-  // value pairs per lane: (3 kq + 1) / 2 pairs of 3 lanes x 2 doubles per slot
-  const size_t pk = kq ? (size_t)(3 * kq + 1) / 2 * 6 * np : 0;
-  A.reserve(&d.f_blk, pk);
-  A.reserve(&d.f_dinv, kq ? 12 * (size_t)np : 0);
-  A.reserve(&d.b_blk, pk);
   int *qfp, *qbp;
   A.reserve(&qfp, S.qf_ptr.size());
   A.reserve(&qbp, S.qb_ptr.size());
@@ -432,6 +445,8 @@ int build(Cloth* c, const cs_mesh* m) {
     dev_free(tmp, s);
     if (st != kOk) return st;
     strip_reset = true;  // once the arrays it reads are uploaded
+  } else if (int st = packed_arrays(c)) {
+    return st;
   }
   CS_HIP(hipMemsetAsync(d.sum.ticket, 0, sizeof(unsigned int), s));
   CS_HIP(hipMemsetAsync(d.sum2.ticket, 0, sizeof(unsigned int), s));
@@ -621,6 +636,7 @@ int cs_cloth_destroy(cs_cloth* p) {
   c->prof.release();
   dev_free(c->sweep_verts, c->stream);
   c->arena.release(c->stream);
+  c->quad.release(c->stream);
   pinned_free(c->hflags);
   pinned_free(c->hscal);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -645,10 +661,10 @@ int cs_cloth_memory(const cs_cloth* p, long long* bytes) {
   if (!p || !bytes) return kBadArg;
   const Cloth* c = H(p);
   const ContactState& k = c->contact;
-  // the arena, the contact records at their current capacity (keys, tests,
+  // the arenas, the contact records at their current capacity (keys, tests,
   // leaf pairs, two sort buffers, groups, the set, impulse links), sort
   // scratch and the per-vertex contact arrays
-  *bytes = (long long)c->arena.bytes() + (long long)k.cap * 88 + (long long)k.tmp_bytes +
+  *bytes = (long long)(c->arena.bytes() + c->quad.bytes()) + (long long)k.cap * 88 + (long long)k.tmp_bytes +
            (long long)k.geom_cap * 128 +
            (long long)c->S.np * 64;
   return kOk;
@@ -827,6 +843,8 @@ int cs_set_option(cs_cloth* p, int option, int value) {
       set_error("the row-by-row sweep is FP64 only: set CS_OPT_PRECISION to 0 first");
       return kBadArg;
     }
+    if (value == 1)
+      if (int st = packed_arrays(c)) return st;
     c->d.sweep_variant = value;
     return kOk;
   }
@@ -835,6 +853,8 @@ int cs_set_option(cs_cloth* p, int option, int value) {
       set_error("the one-workgroup PCG solve needs the packed sweep, FP64 and 3 np <= 65536");
       return kBadArg;
     }
+    if (value == 2)
+      if (int st = packed_arrays(c)) return st;
     c->d.pcg_variant = value;
     return kOk;
   }
@@ -1350,6 +1370,11 @@ extern "C" int cs_batch_step(cs_batch* p, int nsteps, cs_step_stats* stats) {
       return kBadArg;
     }
   hipStream_t s = b->stream;
+  b->view.strips = b->view.piped;
+  for (Cloth* c : b->cl) b->view.strips = b->view.strips && strips_ok(c->d);
+  if (!b->view.strips)  // a member without a strip plan: none by strips
+    for (Cloth* c : b->cl)
+      if (int st = packed_arrays(c)) return st;
   // member cloths may have pending work on their own streams
   for (Cloth* c : b->cl) CS_HIP(hipStreamSynchronize(c->stream));
   if (int st = batch_refresh(b)) return st;
@@ -1357,8 +1382,6 @@ extern "C" int cs_batch_step(cs_batch* p, int nsteps, cs_step_stats* stats) {
   // same either way): the one-workgroup solve when every member selects it
   b->view.wg = b->view.piped;
   for (Cloth* c : b->cl) b->view.wg = b->view.wg && pcg_wg_ok(c->d) && c->d.pcg_variant == 2;
-  b->view.strips = b->view.piped;
-  for (Cloth* c : b->cl) b->view.strips = b->view.strips && strips_ok(c->d);
   // one sweep instance serves every member: their coefficient formats agree
   b->view.f32 = b->cl[0]->d.precision != 0;
   for (Cloth* c : b->cl)

@@ -174,6 +174,33 @@ def test_factor_by_strips_bitwise(sim_mod, oracle_mod, name):
             assert np.array_equal(fd, wd) and np.array_equal(fc, wc)
 
 
+def test_packed_factor_is_allocated_when_a_solve_needs_it(sim_mod):
+    """A cloth that is swept by strips does not hold the packed factor of the
+    one-workgroup sweeps (per vertex and sweep 3 K values in pairs of 6, and
+    12 doubles) until an option or a batch asks for such a solve."""
+    cl = _grid(17, 33)
+    with sim_mod.DeviceCloth(cl) as d, sim_mod.DeviceCloth(_mesh("shuffled20")) as rows, \
+            sim_mod.DeviceCloth(cl) as e:
+        m = d.memory()
+        want = (2 * ((3 * 6 + 1) // 2) * 6 + 12) * 8 * cl.np_
+        d.ilu_factor()
+        d.ilu_solve(cl.xyz)
+        assert d.memory() == m
+        d.set_option(2, 2)
+        assert 0 <= d.memory() - m - want < 3 * 256
+        m2 = d.memory()
+        d.set_option(2, 0)
+        d.set_option(1, 1)
+        assert d.memory() == m2
+        m = e.memory()
+        with sim_mod.DeviceBatch([e]) as b:
+            b.step(1)
+        grown = e.memory()  # by the contact buffers
+        with sim_mod.DeviceBatch([e, rows]) as b:
+            b.step(1)
+        assert 0 <= e.memory() - grown - want < 3 * 256
+
+
 def _states(devs):
     return [a for d in devs for a in d.get_state()]
 
