@@ -16,7 +16,7 @@ cloth's setup does not hold back the admission of the ones after it.
 
 Admission is by resident device footprint: a request is admitted once it has
 arrived and its estimated footprint (BYTES_PER_VERTEX_ESTIMATE per vertex, or
-the measured ``cs_cloth_memory`` once created) fits the HBM budget beside the
+the measured ``cs_cloth_memory`` once created and after each step) fits the HBM budget beside the
 resident ones.  A request that can never fit, whose cloth cannot be created,
 whose step fails or whose solve turns non-finite gets an error result while
 the others continue.  Requests can be cancelled (``Server.cancel``) or evicted
@@ -73,8 +73,14 @@ from .scene import Cloth, SplitMix64
 from .sim import DeviceBatch, DeviceCloth
 
 # admission estimate before a cloth exists on the device: bytes per vertex of
-# the resident footprint (measured ~5.5 KB/vertex at 65k vertices, rounded up)
-BYTES_PER_VERTEX_ESTIMATE = 8192
+# the resident footprint (cs_cloth_memory of grids at creation: 9956 at 65k
+# vertices, 9940 at 100k, 9920 at 1M, rounded up).  The real footprint counts
+# from the creation on, and again after each step (contact buffers grow: 10151,
+# 10414 and 10990 after a step of the same cloths).
+BYTES_PER_VERTEX_ESTIMATE = 10240
+# a request is refused only where this much does not fit the budget; between
+# the two it is admitted when nothing else is resident
+LEAST_BYTES_PER_VERTEX = 8192
 
 # lane boundaries by vertex count: six lanes, [0, 2500), [2500, 8000), ...,
 # [60000, inf).  A lane's tick lasts as long as its slowest member's step, so
@@ -301,6 +307,12 @@ class _Lane:
         a.impulse_applied.append(bool(st["impulse_applied"]))
         a.n_prox.append(int(st["n_prox"]))
         a.n_ccd.append([int(c) for c in st["n_ccd"][:st["n_ccd_pass"]]])
+        # contact buffers grow with the contacts met: admission counts them
+        mem = a.dev.memory()
+        if mem > a.memory:
+            with self.server.cv:
+                self.server.resident += mem - a.memory
+                a.memory = mem
 
     def _run_solo(self):
         """Step one cloth alone (its own stream) until it finishes, fails, is
@@ -536,7 +548,7 @@ class Server:
         try:
             with self.cv:
                 for a in list(self.pending):
-                    need = a.req.cloth.np_ * BYTES_PER_VERTEX_ESTIMATE
+                    need = a.req.cloth.np_ * LEAST_BYTES_PER_VERTEX
                     if need > self.budget:
                         self.pending.remove(a)
                         self.live.discard(id(a))

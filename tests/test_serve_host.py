@@ -20,6 +20,7 @@ class FakeCloth:
     fail_create = set()   # cloth names whose creation fails
     oom_once = set()      # cloth names whose first creation runs out of memory
     nonfinite_at = {}     # cloth name -> step index whose solve turns non-finite
+    grows = {}            # cloth name -> bytes per vertex once stepped
     lock = threading.Lock()
 
     def __init__(self, cloth):
@@ -38,7 +39,7 @@ class FakeCloth:
         self.closed = False
 
     def memory(self):
-        return self.np_ * 4096
+        return self.np_ * (FakeCloth.grows.get(self.cloth.name, 4096) if self.k else 4096)
 
     def set_option(self, option, value):
         self.option = (option, value)
@@ -104,6 +105,7 @@ def fake(monkeypatch):
     FakeCloth.fail_create = set()
     FakeCloth.oom_once = set()
     FakeCloth.nonfinite_at = {}
+    FakeCloth.grows = {}
     FakeBatch.tick_s = 0.001
     FakeBatch.ticks = []
     return FakeCloth
@@ -233,6 +235,33 @@ def test_tight_budget_queues_and_out_of_memory_retries(fake):
     for q in reqs:
         _check({r.rid: r for r in out["results"]}[q.rid], q)
     assert fake.created.count("c1") == 1  # the out-of-memory creation was retried
+
+
+@pytest.mark.parametrize("solo", [False, True])
+def test_growth_of_a_stepped_cloth_counts_against_the_budget(fake, solo):
+    """A cloth whose contact buffers grow past the estimate takes the room of
+    the request that arrives later: that one waits until the first is done."""
+    est = 12 * 12 * serve.BYTES_PER_VERTEX_ESTIMATE
+    fake.grows["c0"] = 3 * serve.BYTES_PER_VERTEX_ESTIMATE // 2
+    reqs = [_req(0, 12, 60), _req(1, 12, 4)]
+    reqs[1].arrival = 0.1
+    FakeBatch.tick_s = 0.01
+    srv = serve.Server(2 * est + 1, lanes=(), solo_from=1 if solo else None)
+    out = srv.run(reqs, realtime=True)
+    assert not out["failures"] and len(out["results"]) == 2
+    by = {r.rid: r for r in out["results"]}
+    assert by[1].admitted_s >= by[0].finished_s
+    assert srv.resident == 0
+
+
+def test_request_between_the_least_footprint_and_the_estimate_runs_alone(fake):
+    n = 12 * 12
+    assert serve.LEAST_BYTES_PER_VERTEX < serve.BYTES_PER_VERTEX_ESTIMATE
+    out = serve.Server(n * serve.LEAST_BYTES_PER_VERTEX, lanes=()).run(
+        [_req(0, 12, 4), _req(1, 12, 3), _req(2, 13, 1)], realtime=False)
+    assert [f.rid for f in out["failures"]] == [2]
+    assert sorted(r.rid for r in out["results"]) == [0, 1]
+    assert all(len(names) == 1 for _, _, names in FakeBatch.ticks)
 
 
 def test_nonfinite_step_fails_only_that_request(fake):
