@@ -6,6 +6,7 @@
 #include <atomic>
 #include <climits>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -138,6 +139,7 @@ struct Cloth {
   Params P;
   DevCloth d;
   Arena arena;
+  Arena strips;  // the strip plan's records, where the mesh has one
   Arena quad;  // the packed factor of the one-workgroup sweeps, once needed (packed_arrays)
   hipStream_t stream = nullptr;
   int* hflags = nullptr;  // pinned
@@ -329,23 +331,37 @@ int build(Cloth* c, const cs_mesh* m) {
       72LL * nnz >= (1LL << 31))
     T.ok = false;
   int *stfp, *stbp, *stfs, *stbs, *stfr, *stbr, *stsl;
-  const size_t nsf = T.ok ? T.fwd.nsub + kStripTail : 0, nsb = T.ok ? T.bwd.nsub + kStripTail : 0;
-  A.reserve(&stfp, T.fwd.ptr.size());
-  A.reserve(&stbp, T.bwd.ptr.size());
-  A.reserve(&stfs, 64 * nsf);
-  A.reserve(&stbs, 64 * nsb);
-  A.reserve(&stfr, kStripRows * nsf);
-  A.reserve(&stbr, kStripRows * nsb);
-  A.reserve(&stsl, T.ok ? (size_t)np : 0);
-  A.reserve(&d.st_frec, strip_record_bytes(true, T.k) * nsf);
-  A.reserve(&d.st_brec, strip_record_bytes(false, T.k) * nsb);
-  A.reserve(&d.st_sb, 64 * nsb);
-  A.reserve(&d.st_ticket, 2);
   int* strows;
-  A.reserve(&strows, 8 * kStripRows * nsf);
   double* host_pd;
   A.reserve(&host_pd, 4 * (size_t)np);
   if (int st = A.commit(c->stream)) return st;
+  if (T.ok) {
+    const size_t nsf = T.fwd.nsub + kStripTail, nsb = T.bwd.nsub + kStripTail;
+    Arena B;
+    B.reserve(&stfp, T.fwd.ptr.size());
+    B.reserve(&stbp, T.bwd.ptr.size());
+    B.reserve(&stfs, 64 * nsf);
+    B.reserve(&stbs, 64 * nsb);
+    B.reserve(&stfr, kStripRows * nsf);
+    B.reserve(&stbr, kStripRows * nsb);
+    B.reserve(&stsl, (size_t)np);
+    B.reserve(&d.st_frec, strip_record_bytes(true, T.k) * nsf);
+    B.reserve(&d.st_brec, strip_record_bytes(false, T.k) * nsb);
+    B.reserve(&d.st_sb, 64 * nsb);
+    B.reserve(&d.st_ticket, 2);
+    B.reserve(&strows, 8 * kStripRows * nsf);
+    // A ribbon's sub-levels hold a few rows each, so its records can take ten
+    // times the packed factor (9.6 KB per vertex at 5000 x 3).  Where there is
+    // no memory for them, or they are more than CLOTHSIM_STRIP_BYTES, the
+    // sweeps go by the packed factor.
+    const char* most = std::getenv("CLOTHSIM_STRIP_BYTES");
+    if ((most && B.bytes() > std::strtoull(most, nullptr, 10)) || B.commit(c->stream) != kOk) {
+      (void)hipGetLastError();
+      T.ok = false;
+    } else {
+      c->strips = B;
+    }
+  }
   d.tri = tri;
   d.quad = quad;
   d.bc = bc;
@@ -636,6 +652,7 @@ int cs_cloth_destroy(cs_cloth* p) {
   c->prof.release();
   dev_free(c->sweep_verts, c->stream);
   c->arena.release(c->stream);
+  c->strips.release(c->stream);
   c->quad.release(c->stream);
   pinned_free(c->hflags);
   pinned_free(c->hscal);
@@ -664,7 +681,7 @@ int cs_cloth_memory(const cs_cloth* p, long long* bytes) {
   // the arenas, the contact records at their current capacity (keys, tests,
   // leaf pairs, two sort buffers, groups, the set, impulse links), sort
   // scratch and the per-vertex contact arrays
-  *bytes = (long long)(c->arena.bytes() + c->quad.bytes()) + (long long)k.cap * 88 + (long long)k.tmp_bytes +
+  *bytes = (long long)(c->arena.bytes() + c->strips.bytes() + c->quad.bytes()) + (long long)k.cap * 88 + (long long)k.tmp_bytes +
            (long long)k.geom_cap * 128 +
            (long long)c->S.np * 64;
   return kOk;

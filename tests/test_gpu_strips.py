@@ -174,6 +174,23 @@ def test_factor_by_strips_bitwise(sim_mod, oracle_mod, name):
             assert np.array_equal(fd, wd) and np.array_equal(fc, wc)
 
 
+def test_no_room_for_the_records_is_not_an_error(sim_mod, monkeypatch):
+    """A cloth whose strip records do not fit is created without a plan and
+    steps to the same state."""
+    cl = _grid(60, 3)
+    cl.pcg_maxit = 30
+    states = []
+    for most in (None, "100000", "1"):
+        if most:
+            monkeypatch.setenv("CLOTHSIM_STRIP_BYTES", most)
+        with sim_mod.DeviceCloth(cl) as d:
+            assert bool(d.strip_shape()["strips"]) == (most is None)
+            d.step(2)
+            states.append(_states([d]))
+    for got in states[1:]:
+        assert all(np.array_equal(g, w) for g, w in zip(got, states[0]))
+
+
 def test_packed_factor_is_allocated_when_a_solve_needs_it(sim_mod):
     """A cloth that is swept by strips does not hold the packed factor of the
     one-workgroup sweeps (per vertex and sweep 3 K values in pairs of 6, and
