@@ -65,6 +65,13 @@ def test_items_equal_the_loop(sim_mod, kind, n):
     assert np.array_equal(sim_mod.ordered_sum(t), _sequential(t), equal_nan=True)
 
 
+@pytest.mark.parametrize("name", ["at the cap", "past the cap", "full windows"])
+def test_tiles_with_as_many_items_as_fit(sim_mod, name):
+    from test_item_sum_emulation import crafted
+    t = crafted()[name]
+    assert sim_mod.ordered_sum(t) == _sequential(t)
+
+
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan, 1.7e308])
 @pytest.mark.parametrize("at", [0, 1023, 1500, 70000])
 def test_special_values(sim_mod, bad, at):

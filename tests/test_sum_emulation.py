@@ -141,10 +141,10 @@ def wave_burst(buf, m, len_, s, bnd):
         w = wn
 
 
-def wave_walk(buf, len_, s, bnd):
+def wave_walk(buf, len_, s, bnd, first=0):
     lo52, hi53 = TWO52 + 1.0, 2.0 * TWO52 - 1.0
     lanes = np.arange(64)
-    pos = 0
+    pos = first
     while pos < len_:
         if math.isnan(s):
             break
