@@ -573,8 +573,7 @@ int internal_step(Cloth* c, double* conv, int* iters) {
   c->have_x1 = true;
   Prof* prof = c->prof.on ? &c->prof : nullptr;
   if (int st = launch_assemble(d, c->P, s, prof)) return st;
-  if (int st = launch_ilu(d, s, prof)) return st;
-  c->packed = 0;
+  if (int st = launch_ilu(d, &c->packed, true, s, prof)) return st;
   if (int st = run_pcg(d, c->P.pcg_tol, c->P.pcg_maxit, c->hflags, &c->packed, s, c->poll, prof))
     return st;
   if (int st = launch_finish_internal(d, c->P, s)) return st;
@@ -983,8 +982,7 @@ int cs_ilu_factor(cs_cloth* p, int* n_singular) {
   if (!p) return kBadArg;
   Cloth* c = H(p);
   CS_HIP(hipMemsetAsync(c->d.flags, 0, sizeof(int) * kNumFlag, c->stream));
-  if (int st = launch_ilu(c->d, c->stream)) return st;
-  c->packed = 0;
+  if (int st = launch_ilu(c->d, &c->packed, false, c->stream)) return st;
   CS_HIP(hipMemcpyAsync(c->hflags, c->d.flags, sizeof(int) * kNumFlag, hipMemcpyDeviceToHost, c->stream));
   if (int st = sync(c)) return st;
   if (int st = check_solve(c)) return st;

@@ -1472,8 +1472,14 @@ int launch_assemble(const DevCloth& c, const Params& P, hipStream_t s, Prof* pro
   return kOk;
 }
 
-int launch_ilu(const DevCloth& c, hipStream_t s, Prof* prof) {
+// this cloth's solve goes by strips
+static bool solve_by_strips(const DevCloth& c) {
+  return !(pcg_wg_ok(c) && c.pcg_variant == 2) && strips_ok(c);
+}
+
+int launch_ilu(const DevCloth& c, int* packed, bool solve, hipStream_t s, Prof* prof) {
   ProfScope ps(prof, kProfFactor);
+  *packed = 0;
   // By strips where the mesh fits them; else one workgroup walks the levels.
   // Both, whole launch: 256^2 sheet 4.6 and 14.4 ms, 128^2 2.3 and 4.2
   // ms, 32^2 0.54 and 0.68 ms.
@@ -1494,14 +1500,15 @@ int launch_ilu(const DevCloth& c, hipStream_t s, Prof* prof) {
   }
   hipLaunchKernelGGL(k_ilu_redo<One>, dim3(1), dim3(1024), 0, s, One{c, {}});
   CS_HIP(hipGetLastError());
-  return kOk;
+  return solve ? ensure_packed(c, solve_by_strips(c), packed, s) : kOk;
 }
 
 int ensure_packed(const DevCloth& c, bool strips, int* packed, hipStream_t s) {
   const int want = strips ? kPackedStrips : kPackedQuad;
   if (*packed & want) return kOk;
+  if (int st = strips ? launch_strip_pack(c, s) : launch_pack_factor(c, s)) return st;
   *packed |= want;
-  return strips ? launch_strip_pack(c, s) : launch_pack_factor(c, s);
+  return kOk;
 }
 
 int launch_pack_factor(const DevCloth& c, hipStream_t s) {
@@ -1534,12 +1541,9 @@ int run_pcg(const DevCloth& c, double tol, int maxit, int* host_flags, int* pack
             int poll, Prof* prof) {
   const long n3 = 3L * c.np;
   const bool wg = pcg_wg_ok(c) && c.pcg_variant == 2;
-  const bool strips = !wg && strips_ok(c);
+  const bool strips = solve_by_strips(c);
   const int layout = strips ? kRhsStrips : c.fslot ? kRhsQuad : kRhsRows;
-  {
-    ProfScope ps(prof, kProfOther);
-    if (int st = ensure_packed(c, strips, packed, s)) return st;
-  }
+  if (int st = ensure_packed(c, strips, packed, s)) return st;
   if (wg) {
     ProfScope ps(prof, kProfPcgWg);
     launch_pcg_wg(c.kpack, dim3(1), One{c, {}}, tol * tol, maxit, s);

@@ -23,8 +23,9 @@ int ilu_stage_blocks(int widest_row);
 int launch_bend_setup(const DevCloth& c, const Params& P, hipStream_t s);
 // element kernels + gather assembly of A and b (after boundary conditions)
 int launch_assemble(const DevCloth& c, const Params& P, hipStream_t s, Prof* prof = nullptr);
-// copy A into the factor storage and factorise in place
-int launch_ilu(const DevCloth& c, hipStream_t s, Prof* prof = nullptr);
+// block ILU(0) of the assembled system; *packed: the packed copies are stale,
+// and with `solve` the one that this cloth's solve needs is made
+int launch_ilu(const DevCloth& c, int* packed, bool solve, hipStream_t s, Prof* prof = nullptr);
 // rearrange the factor for the packed sweeps (after any change of fdia/fcrs)
 int launch_pack_factor(const DevCloth& c, hipStream_t s);
 // sweeps by strips (cs_strips.hip): one wave per strip of rows.  strips_ok:

@@ -251,6 +251,28 @@ def test_profile_modes(sim_mod):
             sim_mod.check(_lib.load().cs_profile_enable(d.h, 3))
 
 
+@pytest.mark.parametrize("pcg", [0, 2])
+def test_profile_classes_are_the_same_alone_and_in_a_batch(sim_mod, pcg):
+    """A step's launches fall into the same classes alone and in a batch (the
+    packing of the factor counts as factorisation in both)."""
+    cl = scene.fold_sweep(24, size=0.3)
+    cl.pcg_maxit = 20
+    with sim_mod.DeviceCloth(cl) as d:
+        d.set_option(2, pcg)
+        d.profile(True)
+        d.step(1)
+        alone = {k: n for k, (ms, n) in d.profile_read().items()}
+        d.profile(False)
+        d.set_state(cl.xyz, cl.uvw)
+        d.time = 0.0
+        with sim_mod.DeviceBatch([d]) as b:
+            b.profile(True)
+            b.step(1)
+            batch = {k: n for k, (ms, n) in b.profile_read().items()}
+    assert alone.pop("contact") == 1 and batch.pop("contact") == 0  # run per cloth, not shared
+    assert alone == batch and alone["ilu_factor"] == 1
+
+
 @pytest.mark.parametrize("nsing", [5, 14])
 def test_ilu_singular_pivots(sim_mod, oracle_mod, nsing):
     """Exactly singular pivots: rows whose diagonal block and lower blocks are
