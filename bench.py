@@ -6,20 +6,22 @@ Headline: the serving stream.  N requests arrive as a Poisson process; each
 is a rectangular cloth whose triangle count is log-uniform in [1e3, 2e5]
 (aspect 1..4), dropped from a seeded height onto its own sphere or box, with
 dt 0.01 and ILU(0)-PCG at tolerance 1e-6 / cap 1000.  Each request runs
-min(drawn steps, K) steps (drawn uniformly in 50..300; the cap bounds the
-run time and is written into `config`).  One step is one StepTime
+two of its drawn steps (50..300, uniform; the cap bounds the run time and is
+written into `config`), and the K timed steps are K / 2 such streams one after
+another, of consecutive seeds, each with the requests of its own (the last one
+with one step if K is odd).  One step is one StepTime
 (self_contact_sparse/main.cpp:213-263): assembly, ILU(0), ILU-PCG, proximity
 + continuous contact pass, post-contact velocity update, in FP64 and
 bit-identical to the reference.
 
 The stream is served with continuous batching (cloth_sim_self_collision_amd.
 serve.Server: HBM admission, size lanes stepping their resident cloths
-together), then the same requests run one after another with the plain
-single-cloth step; `value` is the served whole-job vertex-steps/s (inputs
+together), then the first stream's requests run one after another with the plain
+single-cloth step; `value` is the served whole-job vertex-steps/s over all streams (inputs
 resident once admitted; cloth creation on admission is inside the timed
 run, for both legs), `plain` the plain one, with per-step p50/p99 latencies.
-Every served result is compared bit for bit with the plain one, and the
-first step of each request in the CPU sample with the reference's own code
+Every served result of the first stream is compared bit for bit with the plain
+one, and the first step of each request in the CPU sample with the reference's own code
 (`pos_err_m`).
 
 `roofline`: the kernel class with the most device time in the served run
@@ -57,11 +59,12 @@ HBM_PEAK_GBS = 8000.0
 # scaled by what the counter reads for k_stream_copy of known size; the passes
 # and the scaling are in profiles/
 TRAFFIC_RATIO: dict = {
-    # profiles/fold256_hbm_traffic_pmc.md: (67342.1 * 2.000 + 7171.0) KiB / 59.98 MB
-    ("fold256", "ilu_sweep"): 2.422,
-    # profiles/served_stream_hbm_traffic_pmc.md: batched sweeps, 2.320 + 0.123
-    ("served", "ilu_sweep"): 2.443,
+    # profiles/fold256_hbm_traffic_pmc.md: (67342.1 * 2.000 + 7171.0) KiB / 58.41 MB
+    ("fold256", "ilu_sweep"): 2.487,
+    # profiles/served_stream_hbm_traffic_pmc.md: batched sweeps, 2.382 + 0.126
+    ("served", "ilu_sweep"): 2.508,
 }
+STREAM_STEPS = 2  # steps of each request of a served stream
 METRIC = "vertex-steps/s + p99 step latency, served vs plain GPU, at ≤1e-5 m pos err"
 
 
@@ -71,14 +74,14 @@ def algorithmic_bytes(kind: str, np_: int, nnz: int) -> float:
     mat = 72.0 * (nnz + np_)          # off-diagonal + diagonal 3x3 blocks
     idx = 4.0 * nnz + 4.0 * (np_ + 1)  # column indices + row offsets
     vec = 24.0 * np_                  # one 3-vector per vertex
-    if kind == "ilu_sweep":           # L, U, D^-1 + diagonal index + level rows; r in, z and r.*z out
-        return mat + idx + 12.0 * np_ + 3 * vec
-    if kind == "spmv":                # A; z, p_old in; p, Ap, p.*Ap out
-        return mat + idx + 5 * vec
-    if kind == "pcg_reduce":          # the product vector
-        return vec
-    if kind == "vector_update":       # r, Ap, x, p in; r, x, r.*r out
-        return 7 * vec
+    if kind == "ilu_sweep":           # L, U, D^-1 + diagonal index + level rows; r in, z out
+        return mat + idx + 12.0 * np_ + 2 * vec
+    if kind == "spmv":                # A; z, p_old in; p, Ap out
+        return mat + idx + 4 * vec
+    if kind == "pcg_reduce":          # the two vectors of (p, Ap), or of (r, z) and (r, r)
+        return 2 * vec
+    if kind == "vector_update":       # r, Ap, x, p in; r, x out
+        return 6 * vec
     if kind == "ilu_factor":          # A in, factor out, indices
         return 2 * mat + idx + 12.0 * np_
     return 0.0
@@ -87,7 +90,7 @@ def algorithmic_bytes(kind: str, np_: int, nnz: int) -> float:
 def step_bytes(kind: str, np_: int, nnz: int, iters: int) -> float:
     """Algorithmic bytes of one cloth's step in a kernel class, given its PCG
     iterations: one factorisation; iters + 1 preconditioner sweeps, matrix
-    products and vector updates; three reductions per iteration; the
+    products and vector updates; two launches of reductions per iteration; the
     one-workgroup solve does all of these in one launch."""
     passes = iters + 1
     if kind == "ilu_factor":
@@ -95,7 +98,7 @@ def step_bytes(kind: str, np_: int, nnz: int, iters: int) -> float:
     if kind in ("ilu_sweep", "spmv", "vector_update"):
         return passes * algorithmic_bytes(kind, np_, nnz)
     if kind == "pcg_reduce":
-        return 3 * passes * algorithmic_bytes(kind, np_, nnz)
+        return 2 * passes * algorithmic_bytes(kind, np_, nnz)
     if kind == "pcg_workgroup":
         return sum(step_bytes(k, np_, nnz, iters) for k in ("ilu_sweep", "spmv", "vector_update",
                                                             "pcg_reduce"))
@@ -211,15 +214,19 @@ def cpu_baseline(jobs: list, processes: int, what: str) -> tuple:
 
 
 def serve_leg(args, copy_gbs) -> dict:
-    """The headline: the served stream and the same requests plain."""
+    """The headline: the served streams and the first one's requests plain."""
     from cloth_sim_self_collision_amd import serve
-    wire = serve.poisson_requests(args.requests, args.rate, seed=args.seed, tri_range=(1.0e3, 2.0e5),
-                                  aspect_range=(1.0, 4.0), step_range=(50, 300),
-                                  pcg_maxit=args.pcg_maxit)
-    drawn = [w["steps"] for w in wire]
-    for w in wire:
-        w["steps"] = min(w["steps"], args.steps)
-    reqs = [serve.parse_request(w, k) for k, w in enumerate(wire)]
+    caps = [min(STREAM_STEPS, args.steps - k) for k in range(0, args.steps, STREAM_STEPS)]
+
+    def stream(k):
+        wire = serve.poisson_requests(args.requests, args.rate, seed=args.seed + k,
+                                      tri_range=(1.0e3, 2.0e5), aspect_range=(1.0, 4.0),
+                                      step_range=(50, 300), pcg_maxit=args.pcg_maxit)
+        drawn = [w["steps"] for w in wire]
+        for w in wire:
+            w["steps"] = min(w["steps"], caps[k])
+        return [serve.parse_request(w, i) for i, w in enumerate(wire)], drawn
+    reqs, drawn = stream(0)
     kw = {"solo_from": None if args.solo_from == 0 else args.solo_from} if args.solo_from >= 0 else {}
     if args.lanes:
         kw["lanes"] = tuple(int(v) for v in args.lanes.split(","))
@@ -237,12 +244,34 @@ def serve_leg(args, copy_gbs) -> dict:
     if args.warmup > 0:
         serve.Server(64 << 30, **kw).run(warm, realtime=False)
         serve.run_plain(warm[:1])
-    print(f"[bench] serve: {len(reqs)} requests, {sum(r.cloth.nt for r in reqs)} triangles, "
-          f"step cap {args.steps}", file=sys.stderr, flush=True)
-    srv = serve.Server(64 << 30, profile=not args.no_profile, **kw)
-    served = srv.run(reqs, realtime=True)
-    print(f"[bench] served in {served['wall_s']:.2f} s ({served['ticks']} ticks)", file=sys.stderr,
-          flush=True)
+    runs, tick_log, vertices = [], [], []
+    for k, cap in enumerate(caps):
+        mine = reqs if k == 0 else stream(k)[0]  # built before its clock starts
+        vertices.append(sum(r.cloth.np_ for r in mine))
+        print(f"[bench] stream {k + 1} of {len(caps)}: {len(mine)} requests, "
+              f"{sum(r.cloth.nt for r in mine)} triangles, {cap} steps each", file=sys.stderr,
+              flush=True)
+        one = serve.Server(64 << 30, profile=not args.no_profile, **kw)
+        out = one.run(mine, realtime=True)
+        print(f"[bench] served in {out['wall_s']:.2f} s ({out['ticks']} ticks)", file=sys.stderr,
+              flush=True)
+        tick_log += one.tick_log
+        lat = [m for r in out["results"] for m in r.step_ms]
+        runs.append((out, lat, sum(r.vertices * len(r.step_ms) for r in out["results"])))
+        if k == 0:
+            srv = one
+        else:
+            out["results"] = []  # only the first stream's states are compared
+    served = dict(runs[0][0])
+    lat = np.array([m for _, ms, _ in runs for m in ms])
+    served["wall_s"] = sum(out["wall_s"] for out, _, _ in runs)
+    served["stream_wall_s"] = [out["wall_s"] for out, _, _ in runs]
+    served["first_vertex_steps_per_s"] = served["vertex_steps_per_s"]
+    served["vertex_steps_per_s"] = sum(v for _, _, v in runs) / served["wall_s"]
+    served["failures"] = [f for out, _, _ in runs for f in out["failures"]]
+    if len(lat):
+        served["p50_step_ms"], served["p99_step_ms"] = (float(v) for v in
+                                                        np.percentile(lat, [50, 99]))
     plain, same = None, None
     if not args.serve_only:
         plain = serve.run_plain(reqs, first_states=True)
@@ -251,8 +280,8 @@ def serve_leg(args, copy_gbs) -> dict:
         same = (not served["failures"] and not plain["failures"] and len(by_rid) == len(reqs) and
                 all(np.array_equal(by_rid[rid].xyz, x) and np.array_equal(by_rid[rid].uvw, v)
                     for rid, x, v in plain["results"]))
-    roof = roofline_from_ticks(srv.tick_log, copy_gbs, "served") if srv.tick_log else None
-    # the served run's timeline: per tick, its lane, start (s), duration (ms),
+    roof = roofline_from_ticks(tick_log, copy_gbs, "served") if tick_log else None
+    # the first stream's timeline: per tick, its lane, start (s), duration (ms),
     # its members' vertex counts and the device time of each kernel class (ms)
     timeline = [[r["lane"], round(r["t0_s"], 3), round(r["ms"], 1), [m[0] for m in r["members"]],
                  {k: round(v[0], 1) for k, v in r["prof"].items() if v[1]}]
@@ -265,7 +294,7 @@ def serve_leg(args, copy_gbs) -> dict:
             "roofline": roof, "timeline": timeline, "req_times": req_times,
             "lane_pcg": srv.lane_pcg, "lane_instances": srv.lane_instances,
             "lane_window": srv.lane_window,
-            "lanes": list(srv.bounds),
+            "lanes": list(srv.bounds), "vertices": vertices, "caps": caps,
             "solo_from": srv.solo_from}
 
 
@@ -442,7 +471,7 @@ def main() -> int:
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=2,
-                    help="steps per request of the served stream (cap on the drawn 50..300)")
+                    help="timed steps: streams of two steps per request, one after another")
     ap.add_argument("--warmup", type=int, default=1)
     ap.add_argument("--requests", type=int, default=64, help="requests of the served stream")
     ap.add_argument("--rate", type=float, default=20.0, help="Poisson arrival rate, 1/s")
@@ -574,7 +603,8 @@ def headline(args, sv, err) -> dict:
                    "tri_range": [1.0e3, 2.0e5], "aspect_range": [1.0, 4.0],
                    "triangles_drawn": [min(nt), max(nt)], "triangles_total": int(sum(nt)),
                    "vertices_total": int(sum(r.cloth.np_ for r in reqs)),
-                   "steps_drawn_range": [50, 300], "step_cap": args.steps,
+                   "streams": len(sv["caps"]), "vertices_per_stream": sv["vertices"],
+                   "steps_drawn_range": [50, 300], "step_cap": sv["caps"][0],
                    "steps_per_request": [r.steps for r in reqs],
                    "dt": reqs[0].cloth.dt, "pcg_tol": reqs[0].cloth.pcg_tol,
                    "pcg_maxit": reqs[0].cloth.pcg_maxit, "lanes_vertex_bounds": sv["lanes"],
@@ -588,8 +618,10 @@ def headline(args, sv, err) -> dict:
         "plain": {"vertex_steps_per_s": plain["vertex_steps_per_s"], "wall_s": plain["wall_s"],
                   "p50_step_ms": plain["p50_step_ms"], "p99_step_ms": plain["p99_step_ms"]}
         if plain else None,
-        "served_wall_s": served["wall_s"],
-        "served_vs_plain": served["vertex_steps_per_s"] / plain["vertex_steps_per_s"] if plain else None,
+        "served_wall_s": served["wall_s"], "stream_wall_s": served["stream_wall_s"],
+        # the same requests: the first stream
+        "served_vs_plain": served["first_vertex_steps_per_s"] / plain["vertex_steps_per_s"]
+        if plain else None,
         "served_equals_plain_bitwise": sv["same"],
         "pos_err_m": err,
         "pos_err_scope": "first step of every request: GPU plain step vs the CPU baseline's step",
