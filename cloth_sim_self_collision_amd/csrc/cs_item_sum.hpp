@@ -22,9 +22,10 @@
 //
 // What bounds it: the chain on one wave, about 8 ns per item and 1.5 us per
 // window of staged items (one summary per tile: 0.6 us per walker step and 6.5
-// ns per addend near every binade change).  Measured, mean of a PCG's
-// reductions with their two launches: 256^2 sheet 108 -> 41 us, 128^2 82 -> 28
-// us, 32^2 33 -> 19 us; 61 x 96 drop 59 -> 24 us.  In these solves one tile in
+// ns per addend near every binade change).  Measured, a PCG's reductions over
+// their number, by events around the launches of one iteration: 256^2 sheet
+// 160 -> 38 us, 128^2 75 -> 22 us, 61 x 96 drop 54 -> 12 us, 32^2 31 -> 10 us
+// ((r, z) and (r, r) share a launch now).  In these solves one tile in
 // 200 to 50000 is walked because a prediction missed.  cs_ordered_sum_noalloc
 // keeps one summary per tile (k_sum_exact): its scratch is a small static array.
 #pragma once

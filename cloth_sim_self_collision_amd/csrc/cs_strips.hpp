@@ -46,7 +46,7 @@ struct StripPlan {
 };
 
 // Strips of s, or ok = false when the mesh does not fit the layout (more than
-// kStripRows imports in reach of a sub-level, a dependency further back than
+// kStripImports imports in reach of a sub-level, a dependency further back than
 // the ring, rows too wide for the packed sweeps).
 void build_strips(const MeshSetup& s, StripPlan& p);
 
